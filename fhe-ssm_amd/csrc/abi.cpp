@@ -1189,7 +1189,7 @@ int ckks_context_memory(const ckks_context* ctx, uint64_t* bytes, uint32_t n) {
     const fhe::Context& c = ctx->c;
     const uint64_t T = c.L + c.K;
     uint64_t v[4] = {0, 0, 0, 0};
-    v[0] = 4 * T * fhe::kN * sizeof(fhe::TwPair) + T * sizeof(fhe::PrimeInfo);
+    v[0] = T * (4 * fhe::kN + 256) * sizeof(fhe::TwPair) + T * sizeof(fhe::PrimeInfo);
     for (auto& kv : c.small_ntt) v[0] += T * kv.first * sizeof(fhe::TwPair);
     for (auto& s : c.scratch) v[1] += s.second;
     for (auto& kv : c.buf_pool) v[2] += kv.first * kv.second.size();

@@ -1,4 +1,5 @@
 // context.cpp -- parameter generation (prime chain, roots, NTT tables) and device upload.
+#include <algorithm>
 #include <hip/hip_runtime.h>
 
 #include <cstring>
@@ -6,6 +7,7 @@
 #include <string>
 
 #include "ckks_engine.h"
+#include "bconv_ntt.hpp"
 #include "engine.hpp"
 
 namespace fhe {
@@ -131,6 +133,7 @@ void context_init(Context& c, const std::vector<uint64_t>& q, const std::vector<
     for (uint64_t m : c.moduli)
         if (m >= (1ull << 60) || (m - 1) % (2ull * kN) != 0 || !is_prime_h(m))
             throw std::invalid_argument("modulus is not an NTT prime below 2^60: " + std::to_string(m));
+    c.mf_primes = *std::min_element(c.moduli.begin(), c.moduli.end()) >= kMfMinQ;
     std::vector<TwPair> tw((size_t)T * kN), itw((size_t)T * kN);
     c.psi.resize(T);
     c.primes.resize(T);
@@ -199,6 +202,16 @@ void context_init(Context& c, const std::vector<uint64_t>& q, const std::vector<
     }
     up((void**)&c.d_twb, twb.data(), twb.size() * sizeof(TwPair));
     up((void**)&c.d_itwb, itwb.data(), itwb.size() * sizeof(TwPair));
+    std::vector<TwPair> twa((size_t)T * 256);
+    for (uint32_t i = 0; i < T; i++) {
+        const TwPair* t = tw.data() + (size_t)i * kN;
+        TwPair* a = twa.data() + (size_t)i * 256;
+        std::copy(t, t + 16, a);
+        for (uint32_t s = 4; s < 8; s++)
+            for (uint32_t n = 0; n < 16; n++)
+                for (uint32_t j = 0; j < (1u << (s - 4)); j++) a[(1u << s) + 16 * j + n] = t[(1u << s) + (n << (s - 4)) + j];
+    }
+    up((void**)&c.d_twa, twa.data(), twa.size() * sizeof(TwPair));
     up((void**)&c.d_primes, c.primes.data(), c.primes.size() * sizeof(PrimeInfo));
 }
 
@@ -241,10 +254,12 @@ void context_release(Context& c) {
     (void)hipFree(c.d_itw);
     (void)hipFree(c.d_twb);
     (void)hipFree(c.d_itwb);
+    (void)hipFree(c.d_twa);
     (void)hipFree(c.d_primes);
     for (auto& kv : c.job_cache) (void)hipFree(kv.second.first);
     prof_clear(c);
     for (auto& kv : c.bconv_cache) (void)hipFree(kv.second.d_tab);
+    for (auto& kv : c.mf_cache) (void)hipFree(kv.second.dev);
     for (auto& s : c.scratch) (void)hipFree(s.first);
     for (auto& kv : c.small_ntt) (void)hipFree(kv.second);
     c.small_ntt.clear();
@@ -268,8 +283,9 @@ void context_release(Context& c) {
     c.side_out = nullptr;
     c.job_cache.clear();
     c.bconv_cache.clear();
+    c.mf_cache.clear();
     c.scratch.clear();
-    c.d_tw = c.d_itw = c.d_twb = c.d_itwb = nullptr;
+    c.d_tw = c.d_itw = c.d_twb = c.d_itwb = c.d_twa = nullptr;
     c.d_primes = nullptr;
 }
 

@@ -34,6 +34,15 @@ struct PrimeInfo {
     uint64_t pmod, rpinv, rpinv_p;
 };
 
+// How an inverse transform ends for one prime (JobSpec.scale).  mode 0: as without.  1 or 2: the limb is stored
+// column-major within 16 rows (word c + 256 r at 4096 (r / 16) + 16 c + r % 16); 1: times a factor c of the caller's that ninv and w1ninv carry (N^-1 c and
+// w_1 N^-1 c with Shoup companions), as digit words: with v the scaled canonical residue, (v + 0x80..80) ^ 0x80..80, the
+// eight signed base-256 digits of v -- what the matrix-core basis conversion reads (bconv_ntt.hip).
+struct InvScale {
+    TwPair ninv, w1ninv;
+    uint64_t mode;
+};
+
 // One limb to transform: offset (in units of N words) from the base pointer, and its prime index.
 struct Job {
     uint32_t off, prime;
@@ -63,6 +72,8 @@ struct JobSpec {
     // a negative value) into limb l's prime: a rescale's dropped limb spread over the kept ones.
     const uint64_t* lift;
     uint64_t lift_pstride, lift_q;
+    // Inverse transforms (two-pass mode only): how the limbs end, by prime [L+K], or null
+    const InvScale* scale;
 };
 
 enum class NttMode { TwoPass = 0, Fused = 1 };
@@ -81,6 +92,24 @@ struct BConvPlan {
                                 // halves ((v >> 30) << 32 | v mod 2^30)
 };
 
+// The matrix-core basis conversions of one ModUp (a conversion per digit) or ModDown (one), fused with the forward NTT's
+// first pass (bconv_ntt.hip): their tables, first as the host words (host_words of them: the inverse NTT's scale table,
+// the output slots, the conversion constants), then the MFMA operands that a kernel expands from them.
+struct MfConv {
+    uint32_t n_in, n_out, n_grp;       // source limbs, outputs, groups of four outputs
+    uint32_t open;                     // bit per group: all primes below 2^56
+    size_t slots_at, cmat_at, tab_at;  // word offsets in the plan's device memory
+    uint64_t in_off, out_off;          // words from a batch item's base
+};
+
+struct MfPlan {
+    uint32_t ks = 1, n_grp = 0;
+    std::vector<MfConv> conv;
+    std::vector<uint64_t> host;
+    size_t words = 0;
+    uint64_t* dev = nullptr;  // null: built for allocation-free calls only (their arena holds the device copy)
+};
+
 // Device memory lent to one call of the allocation-free entry point: the library's static scratch (scratch.hip).
 // Workspace slots and the call's own device tables (NTT job lists, BConv constants not yet in the context's caches)
 // are carved from it in request order; the tables are written into it by a kernel from its arguments (arena_put),
@@ -95,6 +124,7 @@ struct Arena {
     hipStream_t st = nullptr;
     size_t slot_off[kArenaSlots] = {}, slot_bytes[kArenaSlots] = {};
     std::deque<BConvPlan> plans;  // the call's BConv plans whose tables live in the arena
+    std::map<uint32_t, uint64_t*> mf;  // device copies of MfPlans made for this call, by plan key
 };
 
 // One profiled launch: HIP events recorded on the launch stream around the kernel, plus the
@@ -119,11 +149,16 @@ struct Context {
     // 13..15, inverse stages with t = 1, 2, 4) stored per 256-word block as [k][lane] (see ntt.hip)
     TwPair* d_twb = nullptr;
     TwPair* d_itwb = nullptr;
+    // [L+K][256]: the forward table's first 256 entries as bconv_ntt.hip reads them, entry 2^s + 2^(s-4) n + j of stages
+    // s = 4..7 at 2^s + 16 j + n
+    TwPair* d_twa = nullptr;
     PrimeInfo* d_primes = nullptr;
     NttMode ntt_mode = NttMode::TwoPass;
     // cached device job lists keyed by a shape string (list, distinct primes in it)
     std::map<std::string, std::pair<Job*, uint32_t>> job_cache;
     std::map<std::string, BConvPlan> bconv_cache;
+    std::map<uint32_t, MfPlan> mf_cache;  // by kind and level
+    bool mf_primes = false;               // every prime is large enough for the matrix-core conversion's reduction
     // per-limb constants of the Q chain with their Shoup companions, computed on first use: P^-1 mod q_i,
     // P R^-1 mod q_i (R = 2^64), P mod q_i, and by j the row q_j^-1 mod q_i (i < j)
     std::vector<TwPair> tab_pinv, tab_pmodr, tab_pmod;
@@ -188,5 +223,7 @@ hipError_t arena_put(void* dst, const void* src, size_t bytes, hipStream_t st);
 
 hipError_t launch_ntt(const Context& ctx, uint64_t* data, const JobSpec& js, uint32_t n_jobs, bool inverse,
                       NttMode mode, hipStream_t st);
+// the forward transform's second pass alone, over limbs that hold the first pass's output as bconv_ntt.hip leaves it
+hipError_t launch_ntt_fwd_b(const Context& ctx, uint64_t* data, const JobSpec& js, uint32_t n_jobs, hipStream_t st);
 
 }  // namespace fhe

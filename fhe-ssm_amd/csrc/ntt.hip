@@ -44,7 +44,8 @@ namespace fhe {
 namespace {
 
 constexpr int kTileThreads = 256;
-constexpr int kLdsWords = 16 * 272;  // one tile, padded to 17 words per 16 (both passes: no bank conflicts)
+constexpr int kLdsWords = 16 * 272;    // one tile, padded to 17 words per 16 (both passes: no bank conflicts)
+constexpr int kLdsWordsCm = 16 * 273;  // and to 273 per block where lanes stand on 16 blocks
 
 __device__ __forceinline__ void job_of(const JobSpec& js, uint32_t u, uint32_t& off, uint32_t& prime) {
     if (js.jobs) {
@@ -217,26 +218,49 @@ __device__ __forceinline__ void fwd_a_tile(uint64_t* __restrict__ a, const TwPai
     for (int k = 0; k < 16; k++) __builtin_nontemporal_store(x[k], &a[col + 256 * (16 * rg + k)]);
 }
 
+// a word at a byte offset from a wave-uniform base (the global_load form with a scalar base and a 32-bit offset)
+__device__ __forceinline__ uint64_t ld_at(const uint64_t* base, uint32_t byte_off) {
+    return *reinterpret_cast<const uint64_t*>(reinterpret_cast<const char*>(base) + byte_off);
+}
+__device__ __forceinline__ uint64_t ld_at_nt(const uint64_t* base, uint32_t byte_off) {
+    return __builtin_nontemporal_load(reinterpret_cast<const uint64_t*>(reinterpret_cast<const char*>(base) + byte_off));
+}
+
 // ---------------------------------------------------------------- forward pass B (256-word blocks)
 // Epi: what becomes of the transformed tile, held transposed in LDS (word rl + 16 k of block b at L[rl + 17 k]) --
 // StoreLimb (the default): stored over the limb; otherwise first = epi.begin(b, rl) before the final reduction and
 // exchange (loads that do not depend on the tile), then epi.end(first, L, b, rl).
+// kCm: the intermediate has each tile's 16 blocks column-major (word w of block b at 4096 (b / 16) + 16 w + b % 16, from
+// bconv_ntt.hip), read with the lanes on the 16 blocks.
 struct StoreLimb {
     struct First {};
 };
 
-template <bool kOpen, class Epi = StoreLimb>
+template <bool kOpen, bool kCm, class Epi = StoreLimb>
 __device__ __forceinline__ void fwd_b_tile(uint64_t* __restrict__ a, const TwPair* __restrict__ tw, const PrimeInfo& P,
                                            int tile, int g, uint64_t* lds, const Epi& epi = Epi{}) {
+    // opaque per instance: otherwise the addresses that the open and the other instance share are formed before their
+    // branch and kept, spilled, through one for the other (the row-major form has the registers: nothing gained there)
+    if (kCm) asm volatile("" : "+v"(g));
     const uint64_t q = P.q;
     const uint64_t q4 = q << 2, nq = 0 - q;
+    constexpr int kBlk = kCm ? 273 : 272;  // LDS words of a block
+    // first half: thread (b1, r1) on words r1 + 16 k of block b1
     const int bl = g >> 4, rl = g & 15;
     const int b = tile * 16 + bl;  // block index within the limb
     uint64_t* blk = a + 256 * b;
-    uint64_t* L = lds + bl * 272;
+    uint64_t* L = lds + bl * kBlk;
+    const int bl1 = kCm ? g & 15 : bl, r1 = kCm ? g >> 4 : rl;
+    const int b1 = kCm ? tile * 16 + bl1 : b;
     uint64_t x[16];
+    if (kCm) {
+        const uint32_t bo = (4096 * tile + 16 * r1 + bl1) * 8;
 #pragma unroll
-    for (int k = 0; k < 16; k++) x[k] = __builtin_nontemporal_load(&blk[rl + 16 * k]);
+        for (int k = 0; k < 16; k++) x[k] = ld_at_nt(a + 256 * k, bo);
+    } else {
+#pragma unroll
+        for (int k = 0; k < 16; k++) x[k] = __builtin_nontemporal_load(&blk[rl + 16 * k]);
+    }
     // stages 8+s, s = 0..3: r = rl + 16k; twiddle 2^(8+s) + b 2^s + (k >> (4-s)), which pass B's table stores at
     // 2^(8+s) + (k >> (4-s)) 256 + b (the four blocks of a wave read adjacent pairs).  All 15 are requested with the
     // data (left to the compiler, each stage's loads were issued just before its butterflies, one exposed L2 round
@@ -245,7 +269,7 @@ __device__ __forceinline__ void fwd_b_tile(uint64_t* __restrict__ a, const TwPai
 #pragma unroll
     for (int s = 0, n = 0; s < 4; s++)
 #pragma unroll
-        for (int j = 0; j < (1 << s); j++, n++) tw03[n] = tw[(256 << s) + (j << 8) + b];
+        for (int j = 0; j < (1 << s); j++, n++) tw03[n] = tw[(256 << s) + (j << 8) + b1];
 #pragma unroll
     for (int s = 0; s < 4; s++) {
         const int h = 8 >> s;
@@ -269,7 +293,7 @@ __device__ __forceinline__ void fwd_b_tile(uint64_t* __restrict__ a, const TwPai
         for (int i = 0; i < (1 << (s - 4)); i++, n++) tw4[n] = tw[(256 << s) + (b << s) + (i << 4) + rl];
     // LDS word index of r: r + (r >> 4)
 #pragma unroll
-    for (int k = 0; k < 16; k++) L[rl + 17 * k] = x[k];
+    for (int k = 0; k < 16; k++) (kCm ? lds + bl1 * kBlk : L)[r1 + 17 * k] = x[k];
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < 8; i++) tw7[i] = tw[(256 << 7) + (b << 7) + (i << 4) + rl];
@@ -316,7 +340,9 @@ struct KsIn {
     size_t xs, es;      // digit strides of the extension (in) and of the key, in words
 };
 
-template <bool kOpen, bool kProd, int kD = 0>
+// kCm: the limb will end column-major within 16 rows (InvScale): this tile's 16 rows are stored in their own 4,096 words
+// (the transform may be in place) by pass A's tiles, word c + 256 b at 4096 (b / 16) + 256 (c / 16) + 16 (b % 16) + c % 16.
+template <bool kOpen, bool kProd, bool kCm, int kD = 0>
 __device__ __forceinline__ void inv_b_tile(uint64_t* a, const uint64_t* in, JobIn ji, const PrimeInfo& P,
                                            const TwPair* __restrict__ tw, int tile, int g, uint64_t* lds,
                                            const KsIn ks = KsIn{}) {
@@ -426,21 +452,30 @@ __device__ __forceinline__ void inv_b_tile(uint64_t* a, const uint64_t* in, JobI
         }
     }
     gs_group_end<kOpen>(x, q);  // the intermediate is stored below 32 q (below 4 q when not open)
+    if constexpr (kCm) {
+        uint64_t* dst = a + 4096 * tile + 16 * bl + rl;
 #pragma unroll
-    for (int k = 0; k < 16; k++) __builtin_nontemporal_store(x[k], &blk[rl + 16 * k]);
+        for (int k = 0; k < 16; k++) __builtin_nontemporal_store(x[k], &dst[256 * k]);
+    } else {
+#pragma unroll
+        for (int k = 0; k < 16; k++) __builtin_nontemporal_store(x[k], &blk[rl + 16 * k]);
+    }
 }
 
 // ---------------------------------------------------------------- inverse pass A (strided columns)
 // GS stages with t = 2^(8+u), u = 0..7: m = 2^(7-u), twiddle m + (r >> (u+1)); then * N^-1.
-template <bool kOpen>
+// kCm (InvScale): the input is as inv_b_tile leaves it with kCm and the limb is stored column-major within 16 rows (over the
+// words the tile read); kDigits: ninv and w1ninv carry a factor of the caller's and the words are stored as digit words.
+template <bool kOpen, bool kCm = false, bool kDigits = false>
 __device__ __forceinline__ void inv_a_tile(uint64_t* __restrict__ a, const TwPair* __restrict__ tw, uint64_t q,
                                            TwPair ninv, TwPair w1ninv, int tile, int g, uint64_t* lds) {
     const uint64_t q4 = q << 2, nq = 0 - q;
-    const int cl = g & 15, rg = g >> 4;
+    int cl = g & 15, rg = g >> 4;
     const int col = tile * 16 + cl;
     uint64_t x[16];
 #pragma unroll
-    for (int k = 0; k < 16; k++) x[k] = __builtin_nontemporal_load(&a[col + 256 * (16 * rg + k)]);
+    for (int k = 0; k < 16; k++)
+        x[k] = __builtin_nontemporal_load(kCm ? &a[4096 * rg + 256 * tile + 16 * k + cl] : &a[col + 256 * (16 * rg + k)]);
     // u = 0..3: r = 16 rg + k, pairs differ in bit u of k; twiddle (128 >> u) + rg 2^(3-u) + (k >> (u+1)).  Those of
     // u = 0, 1 (12 pairs) are requested with the data, not just before their butterflies
     TwPair twa[12];
@@ -463,6 +498,10 @@ __device__ __forceinline__ void inv_a_tile(uint64_t* __restrict__ a, const TwPai
 #pragma unroll
     for (int k = 0; k < 16; k++) lds[(16 * rg + k) * 17 + cl] = x[k];
     __syncthreads();
+    if (kCm) {  // the lanes of a 16 on one column from here on
+        cl = g >> 4;
+        rg = g & 15;
+    }
 #pragma unroll
     for (int k = 0; k < 16; k++) x[k] = lds[(rg + 16 * k) * 17 + cl];
     // u = 4..6: r = rg + 16k, pairs differ in bit (u-4) of k; r >> (u+1) = k >> (u-3)
@@ -486,8 +525,21 @@ __device__ __forceinline__ void inv_a_tile(uint64_t* __restrict__ a, const TwPai
     for (int k = 0; k < 8; k++) {
         const uint64_t X = x[k], Y = x[k + 8];
         const uint64_t v = X + Y;
-        x[k] = (v >> 16) + q - (uint64_t)((uint32_t)v & 0xFFFFu) * cn;
+        x[k] = kDigits ? shoup_lazy4(v, ninv.w, ninv.wp, nq)
+                       : (v >> 16) + q - (uint64_t)((uint32_t)v & 0xFFFFu) * cn;
         x[k + 8] = shoup_lazy4(X + (kOpen ? q << kGs.lg[3][k + 8] : q4) - Y, w1ninv.w, w1ninv.wp, nq);
+    }
+    if constexpr (kCm) {
+#pragma unroll
+        for (int k = 0; k < 16; k++) {
+            uint64_t v = csub_s(k >= 8 || kDigits ? csub_s(x[k], q << 1) : x[k], q);
+            if (kDigits) {
+                constexpr uint64_t kBias = 0x8080808080808080ull;
+                v = (v + kBias) ^ kBias;
+            }
+            __builtin_nontemporal_store(v, &a[4096 * k + 256 * tile + 16 * cl + rg]);
+        }
+        return;
     }
 #pragma unroll
     for (int k = 0; k < 8; k++) __builtin_nontemporal_store(csub_s(x[k], q), &a[col + 256 * (rg + 16 * k)]);
@@ -521,18 +573,21 @@ __global__ __launch_bounds__(kTileThreads) void k_ntt_fwd_a(uint64_t* data, JobS
     }
 }
 
+template <bool kCm>
 __global__ __launch_bounds__(kTileThreads) void k_ntt_fwd_b(uint64_t* data, JobSpec js, const TwPair* tw_all,
                                                            const PrimeInfo* primes) {
-    __shared__ uint64_t lds[kLdsWords];
+    __shared__ uint64_t lds[kCm ? kLdsWordsCm : kLdsWords];
     uint32_t off, prime;
     job_of(js, blockIdx.y, off, prime);
     const PrimeInfo& P = primes[prime];
     if (P.q < kOpenMaxQ)
-        fwd_b_tile<true>(data + (size_t)off * kN, tw_all + (size_t)prime * kN, P, blockIdx.x, threadIdx.x, lds);
+        fwd_b_tile<true, kCm>(data + (size_t)off * kN, tw_all + (size_t)prime * kN, P, blockIdx.x, threadIdx.x, lds);
     else
-        fwd_b_tile<false>(data + (size_t)off * kN, tw_all + (size_t)prime * kN, P, blockIdx.x, threadIdx.x, lds);
+        fwd_b_tile<false, kCm>(data + (size_t)off * kN, tw_all + (size_t)prime * kN, P, blockIdx.x, threadIdx.x, lds);
 }
 
+// kCm (the inverse kernels): with JobSpec.scale (every prime of the jobs has a mode there)
+template <bool kCm>
 __global__ __launch_bounds__(kTileThreads) void k_ntt_inv_b(uint64_t* data, JobSpec js, const TwPair* tw_all,
                                                            const PrimeInfo* primes) {
     __shared__ uint64_t lds[kLdsWords];
@@ -545,13 +600,13 @@ __global__ __launch_bounds__(kTileThreads) void k_ntt_inv_b(uint64_t* data, JobS
     const JobIn ji = js.jobs ? JobIn{nullptr, nullptr} : job_in(js, blockIdx.y);
     if (ji.in2) {
         if (P.q < kGsOpenMaxQ)
-            inv_b_tile<true, true>(a, in, ji, P, tw, blockIdx.x, threadIdx.x, lds);
+            inv_b_tile<true, true, kCm>(a, in, ji, P, tw, blockIdx.x, threadIdx.x, lds);
         else
-            inv_b_tile<false, true>(a, in, ji, P, tw, blockIdx.x, threadIdx.x, lds);
+            inv_b_tile<false, true, kCm>(a, in, ji, P, tw, blockIdx.x, threadIdx.x, lds);
     } else if (P.q < kGsOpenMaxQ) {
-        inv_b_tile<true, false>(a, in, ji, P, tw, blockIdx.x, threadIdx.x, lds);
+        inv_b_tile<true, false, kCm>(a, in, ji, P, tw, blockIdx.x, threadIdx.x, lds);
     } else {
-        inv_b_tile<false, false>(a, in, ji, P, tw, blockIdx.x, threadIdx.x, lds);
+        inv_b_tile<false, false, kCm>(a, in, ji, P, tw, blockIdx.x, threadIdx.x, lds);
     }
 }
 
@@ -564,7 +619,7 @@ struct KsJobArgs {
     uint32_t E, T;
 };
 
-template <int kD>
+template <int kD, bool kCm>
 __global__ __launch_bounds__(kTileThreads) void k_ntt_inv_b_ks(uint64_t* data, JobSpec js, const TwPair* tw_all,
                                                               const PrimeInfo* primes, KsJobArgs ka) {
     __shared__ uint64_t lds[kLdsWords];
@@ -578,9 +633,9 @@ __global__ __launch_bounds__(kTileThreads) void k_ntt_inv_b_ks(uint64_t* data, J
     const TwPair* tw = tw_all + (size_t)prime * kN;
     const JobIn none{nullptr, nullptr};
     if (P.q < kGsOpenMaxQ)
-        inv_b_tile<true, false, kD>(a, xin, none, P, tw, blockIdx.x, threadIdx.x, lds, ks);
+        inv_b_tile<true, false, kCm, kD>(a, xin, none, P, tw, blockIdx.x, threadIdx.x, lds, ks);
     else
-        inv_b_tile<false, false, kD>(a, xin, none, P, tw, blockIdx.x, threadIdx.x, lds, ks);
+        inv_b_tile<false, false, kCm, kD>(a, xin, none, P, tw, blockIdx.x, threadIdx.x, lds, ks);
 }
 
 // k_ntt_inv_b_ks over a key-switch list: item c = pc / 2 has its own extension [kD][E][N] and key
@@ -589,7 +644,7 @@ struct KslJobArgs {
     uint32_t E, T;
 };
 
-template <int kD>
+template <int kD, bool kCm>
 __global__ __launch_bounds__(kTileThreads) void k_ntt_inv_b_ksl(uint64_t* data, JobSpec js, const TwPair* tw_all,
                                                                const PrimeInfo* primes, KslJobArgs ka) {
     __shared__ uint64_t lds[kLdsWords];
@@ -603,23 +658,33 @@ __global__ __launch_bounds__(kTileThreads) void k_ntt_inv_b_ksl(uint64_t* data, 
     const TwPair* tw = tw_all + (size_t)prime * kN;
     const JobIn none{nullptr, nullptr};
     if (P.q < kGsOpenMaxQ)
-        inv_b_tile<true, false, kD>(a, xin, none, P, tw, blockIdx.x, threadIdx.x, lds, ks);
+        inv_b_tile<true, false, kCm, kD>(a, xin, none, P, tw, blockIdx.x, threadIdx.x, lds, ks);
     else
-        inv_b_tile<false, false, kD>(a, xin, none, P, tw, blockIdx.x, threadIdx.x, lds, ks);
+        inv_b_tile<false, false, kCm, kD>(a, xin, none, P, tw, blockIdx.x, threadIdx.x, lds, ks);
 }
 
+template <bool kCm>
 __global__ __launch_bounds__(kTileThreads) void k_ntt_inv_a(uint64_t* data, JobSpec js, const TwPair* tw_all,
                                                            const PrimeInfo* primes) {
     __shared__ uint64_t lds[kLdsWords];
     uint32_t off, prime;
     job_of(js, blockIdx.y, off, prime);
     const PrimeInfo& P = primes[prime];
-    if (P.q < kGsOpenMaxQ)
-        inv_a_tile<true>(data + (size_t)off * kN, tw_all + (size_t)prime * kN, P.q, TwPair{P.ninv, P.ninv_p},
-                         TwPair{P.w1ninv, P.w1ninv_p}, blockIdx.x, threadIdx.x, lds);
-    else
-        inv_a_tile<false>(data + (size_t)off * kN, tw_all + (size_t)prime * kN, P.q, TwPair{P.ninv, P.ninv_p},
-                          TwPair{P.w1ninv, P.w1ninv_p}, blockIdx.x, threadIdx.x, lds);
+    uint64_t* a = data + (size_t)off * kN;
+    const TwPair* tw = tw_all + (size_t)prime * kN;
+    const TwPair ninv{P.ninv, P.ninv_p}, w1ninv{P.w1ninv, P.w1ninv_p};
+    const bool open = P.q < kGsOpenMaxQ;
+    if (kCm && js.scale[prime].mode == 1) {
+        const InvScale sc = js.scale[prime];
+        if (open)
+            inv_a_tile<true, true, true>(a, tw, P.q, sc.ninv, sc.w1ninv, blockIdx.x, threadIdx.x, lds);
+        else
+            inv_a_tile<false, true, true>(a, tw, P.q, sc.ninv, sc.w1ninv, blockIdx.x, threadIdx.x, lds);
+    } else if (open) {
+        inv_a_tile<true, kCm>(a, tw, P.q, ninv, w1ninv, blockIdx.x, threadIdx.x, lds);
+    } else {
+        inv_a_tile<false, kCm>(a, tw, P.q, ninv, w1ninv, blockIdx.x, threadIdx.x, lds);
+    }
 }
 
 // ---------------------------------------------------------------- forward pass B that finishes a ModDown
@@ -648,14 +713,6 @@ struct MdrFuse {
     TwPair pmod[kMaxPmap];  // P mod q_i
     TwPair cfin[kMaxPmap];  // R P^-1 q_{l-1}^-1 mod q_i (R = 2^64), times the caller's factor
 };
-
-// a word at a byte offset from a wave-uniform base (the global_load form with a scalar base and a 32-bit offset)
-__device__ __forceinline__ uint64_t ld_at(const uint64_t* base, uint32_t byte_off) {
-    return *reinterpret_cast<const uint64_t*>(reinterpret_cast<const char*>(base) + byte_off);
-}
-__device__ __forceinline__ uint64_t ld_at_nt(const uint64_t* base, uint32_t byte_off) {
-    return __builtin_nontemporal_load(reinterpret_cast<const uint64_t*>(reinterpret_cast<const char*>(base) + byte_off));
-}
 
 // The combine of one thread's words (lane rl of block blk, words rl + 16 k for k = 8g .. 8g+7), after the transform.
 // kTa: the addends are formed from the product's inputs (else read from the addend).  Every pointer and constant is
@@ -716,7 +773,7 @@ struct MdrEpi {
         return B;
     }
 
-    // L: this group's tile; the tiles of polys 0 and 1 are adjacent (kLdsWords apart)
+    // L: this group's tile; the tiles of polys 0 and 1 are adjacent (kLdsWordsCm apart)
     // out_p = (x_p P^-1 + d_p - T_p) q_{l-1}^-1 as one 128-bit sum per poly, A_p = x_p + P d_p + P (q - T_p) (P a0 and
     // P a1 formed first, so that d_p's products enter the sum already times P), then REDC(A_p) R P^-1 q_{l-1}^-1: one
     // Montgomery reduction and one Shoup product per word instead of four Barrett reductions, two products by
@@ -724,8 +781,8 @@ struct MdrEpi {
     // rest below q < 2^60: A_p < 7 q^2 < q R (REDC's input bound), and the accumulator's cross-product sum (below
     // 2^61.6 a term) stays below 2^64.
     __device__ __forceinline__ void end(First cur, const uint64_t* L, int blk, int rl) const {
-        const uint64_t* L0 = L - g * kLdsWords;
-        const uint64_t* L1 = L0 + kLdsWords;
+        const uint64_t* L0 = L - g * kLdsWordsCm;
+        const uint64_t* L1 = L0 + kLdsWordsCm;
         const size_t po = (size_t)(f.l - 1) * kN;
         uint64_t* out0 = f.out + 2 * c * po + (size_t)i * kN;
         uint64_t* out1 = out0 + po;
@@ -774,10 +831,10 @@ struct MdrEpi {
 };
 
 // grid (16 tiles, B (l-1) jobs), 512 threads; job v = i B + c (limb-major: a limb's evk is shared by the batch)
-template <int kD, bool kTa, bool kPost>
+template <int kD, bool kTa, bool kPost, bool kCm>
 __global__ __launch_bounds__(2 * kTileThreads) __attribute__((amdgpu_waves_per_eu(4))) void k_ntt_fwd_b_mdr(
     uint64_t* T, const TwPair* tw_all, const PrimeInfo* primes, MdrFuse f) {
-    __shared__ uint64_t lds[2 * kLdsWords];
+    __shared__ uint64_t lds[2 * kLdsWordsCm];
     const uint32_t i = uni_div(blockIdx.y, f.B), c = blockIdx.y - i * f.B;
     const uint32_t g = threadIdx.x >> 8, t = threadIdx.x & 255;
     const PrimeInfo& P = primes[i];
@@ -786,23 +843,30 @@ __global__ __launch_bounds__(2 * kTileThreads) __attribute__((amdgpu_waves_per_e
     uint64_t* a = T + ((size_t)(2 * c + g) * (f.l - 1) + i) * kN;
     const TwPair* tw = tw_all + (size_t)i * kN;
     if (P.q < kOpenMaxQ)
-        fwd_b_tile<true>(a, tw, P, blockIdx.x, t, lds + g * kLdsWords, epi);
+        fwd_b_tile<true, kCm>(a, tw, P, blockIdx.x, t, lds + g * kLdsWordsCm, epi);
     else
-        fwd_b_tile<false>(a, tw, P, blockIdx.x, t, lds + g * kLdsWords, epi);
+        fwd_b_tile<false, kCm>(a, tw, P, blockIdx.x, t, lds + g * kLdsWordsCm, epi);
 }
 
-template <int kD>
+template <int kD, bool kCm>
 void launch_b_mdr(dim3 grid, dim3 block, hipStream_t st, uint64_t* T, const TwPair* twb, const PrimeInfo* primes,
                   const MdrFuse& f) {
     // the poly-0 constant (an affine output) is a separate instance: the plain relinearization pays nothing for it
-    if (f.ta && f.has_post)
-        hipLaunchKernelGGL((k_ntt_fwd_b_mdr<kD, true, true>), grid, block, 0, st, T, twb, primes, f);
-    else if (f.ta)
-        hipLaunchKernelGGL((k_ntt_fwd_b_mdr<kD, true, false>), grid, block, 0, st, T, twb, primes, f);
-    else if (f.has_post)
-        hipLaunchKernelGGL((k_ntt_fwd_b_mdr<kD, false, true>), grid, block, 0, st, T, twb, primes, f);
-    else
-        hipLaunchKernelGGL((k_ntt_fwd_b_mdr<kD, false, false>), grid, block, 0, st, T, twb, primes, f);
+    auto k = f.ta ? (f.has_post ? k_ntt_fwd_b_mdr<kD, true, true, kCm> : k_ntt_fwd_b_mdr<kD, true, false, kCm>)
+                  : (f.has_post ? k_ntt_fwd_b_mdr<kD, false, true, kCm> : k_ntt_fwd_b_mdr<kD, false, false, kCm>);
+    hipLaunchKernelGGL(k, grid, block, 0, st, T, twb, primes, f);
+}
+
+// the instance for D digits
+template <bool kCm>
+void launch_b_mdr_d(uint32_t D, dim3 grid, dim3 block, hipStream_t st, uint64_t* T, const TwPair* twb,
+                    const PrimeInfo* primes, const MdrFuse& f) {
+    switch (D) {
+        case 1: launch_b_mdr<1, kCm>(grid, block, st, T, twb, primes, f); break;
+        case 2: launch_b_mdr<2, kCm>(grid, block, st, T, twb, primes, f); break;
+        case 3: launch_b_mdr<3, kCm>(grid, block, st, T, twb, primes, f); break;
+        default: launch_b_mdr<4, kCm>(grid, block, st, T, twb, primes, f); break;
+    }
 }
 
 // ---------------------------------------------------------------- forward pass B that finishes a key-switch list
@@ -852,10 +916,10 @@ struct KslEpi {
         return B;
     }
 
-    // L: this group's tile; the tiles of polys 0 and 1 are adjacent (kLdsWords apart)
+    // L: this group's tile; the tiles of polys 0 and 1 are adjacent (kLdsWordsCm apart)
     __device__ __forceinline__ void end(First cur, const uint64_t* L, int blk, int rl) const {
-        const uint64_t* L0 = L - g * kLdsWords;
-        const uint64_t* L1 = L0 + kLdsWords;
+        const uint64_t* L0 = L - g * kLdsWordsCm;
+        const uint64_t* L1 = L0 + kLdsWordsCm;
         const size_t pw = (size_t)f.l * kN;
         uint64_t* out0 = f.out + 2 * c * pw + (size_t)i * kN;
         uint64_t* out1 = out0 + pw;
@@ -901,10 +965,10 @@ struct KslEpi {
 };
 
 // grid (16 tiles, n l jobs), 512 threads; job v = i n + c (limb-major: a limb's tiles of all items on one XCD)
-template <int kD>
+template <int kD, bool kCm>
 __global__ __launch_bounds__(2 * kTileThreads) __attribute__((amdgpu_waves_per_eu(4))) void k_ntt_fwd_b_ksl(
     uint64_t* y, const TwPair* tw_all, const PrimeInfo* primes, KslFuse f) {
-    __shared__ uint64_t lds[2 * kLdsWords];
+    __shared__ uint64_t lds[2 * kLdsWordsCm];
     const uint32_t i = uni_div(blockIdx.y, f.n), c = blockIdx.y - i * f.n;
     const uint32_t g = threadIdx.x >> 8, t = threadIdx.x & 255;
     const PrimeInfo& P = primes[i];
@@ -912,15 +976,17 @@ __global__ __launch_bounds__(2 * kTileThreads) __attribute__((amdgpu_waves_per_e
     uint64_t* a = y + ((size_t)(2 * c + g) * f.l + i) * kN;
     const TwPair* tw = tw_all + (size_t)i * kN;
     if (P.q < kOpenMaxQ)
-        fwd_b_tile<true>(a, tw, P, blockIdx.x, t, lds + g * kLdsWords, epi);
+        fwd_b_tile<true, kCm>(a, tw, P, blockIdx.x, t, lds + g * kLdsWordsCm, epi);
     else
-        fwd_b_tile<false>(a, tw, P, blockIdx.x, t, lds + g * kLdsWords, epi);
+        fwd_b_tile<false, kCm>(a, tw, P, blockIdx.x, t, lds + g * kLdsWordsCm, epi);
 }
 
 // ---------------------------------------------------------------- forward pass B that finishes a plain ModDown
 // The forward NTT of a ModDown's converted P part y ([n_polys][l] limbs, dense) ends with the combine of k_sub_scale
 // instead of a store of y: out[pc][i] = (x[pc][i] - y[pc][i]) s_i (+ the addend for polys pc % add_div == 0, read at
 // (pc / add_group) add_pstride).  The same words as the NTT followed by k_sub_scale, without y's store and reload.
+// kScaled: y comes times s_i already (the matrix-core conversion folds it in): out = x s_i - y.
+template <bool kScaled>
 struct SubEpi {
     struct First {
         uint64_t xv[4];
@@ -966,7 +1032,8 @@ struct SubEpi {
 #pragma unroll
             for (int k = 0; k < 8; k++) {
                 const int kk = 8 * h + k;
-                uint64_t v = shoup(sub_mod(xv[k], L[rl + 17 * kk], q), s.w, s.wp, q);
+                const uint64_t y = L[rl + 17 * kk];
+                uint64_t v = kScaled ? sub_mod(shoup(xv[k], s.w, s.wp, q), y, q) : shoup(sub_mod(xv[k], y, q), s.w, s.wp, q);
                 if (add) v = add_mod(v, av[k], q);
                 __builtin_nontemporal_store(v,
                                             reinterpret_cast<uint64_t*>(reinterpret_cast<char*>(out) + bo + 128 * kk));
@@ -975,22 +1042,23 @@ struct SubEpi {
     }
 };
 
+template <bool kCm>
 __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(4))) void k_ntt_fwd_b_sub(uint64_t* y, JobSpec js, const TwPair* tw_all,
                                                                const PrimeInfo* primes, CombineArgs ca,
                                                                const uint64_t* x, const uint64_t* add,
                                                                uint64_t* out) {
-    __shared__ uint64_t lds[kLdsWords];
+    __shared__ uint64_t lds[kCm ? kLdsWordsCm : kLdsWords];
     uint32_t off, prime;
     job_of(js, blockIdx.y, off, prime);
     const uint32_t i = uni_div(blockIdx.y, js.n_polys), pc = blockIdx.y - i * js.n_polys;
     const PrimeInfo& P = primes[prime];
-    const SubEpi epi{ca, x, add, out, P, i, pc};
+    const SubEpi<kCm> epi{ca, x, add, out, P, i, pc};
     uint64_t* a = y + (size_t)off * kN;
     const TwPair* tw = tw_all + (size_t)prime * kN;
     if (P.q < kOpenMaxQ)
-        fwd_b_tile<true>(a, tw, P, blockIdx.x, threadIdx.x, lds, epi);
+        fwd_b_tile<true, kCm>(a, tw, P, blockIdx.x, threadIdx.x, lds, epi);
     else
-        fwd_b_tile<false>(a, tw, P, blockIdx.x, threadIdx.x, lds, epi);
+        fwd_b_tile<false, kCm>(a, tw, P, blockIdx.x, threadIdx.x, lds, epi);
 }
 
 // ---------------------------------------------------------------- forward pass B that finishes a scalar combination
@@ -1073,9 +1141,9 @@ __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(4)
     uint64_t* a = y + (size_t)off * kN;
     const TwPair* tw = tw_all + (size_t)prime * kN;
     if (P.q < kOpenMaxQ)
-        fwd_b_tile<true>(a, tw, P, blockIdx.x, threadIdx.x, lds, epi);
+        fwd_b_tile<true, false>(a, tw, P, blockIdx.x, threadIdx.x, lds, epi);
     else
-        fwd_b_tile<false>(a, tw, P, blockIdx.x, threadIdx.x, lds, epi);
+        fwd_b_tile<false, false>(a, tw, P, blockIdx.x, threadIdx.x, lds, epi);
 }
 
 // Fused: one limb per workgroup of 4 x 256 threads; each 256-thread group owns one LDS tile.
@@ -1098,7 +1166,7 @@ __global__ __launch_bounds__(kTileThreads* kFusedGroups) void k_ntt_fwd_fused(ui
         __syncthreads();
     }
     for (int t = grp; t < 16; t += kFusedGroups) {
-        fwd_b_tile<false>(a, twb_all + (size_t)prime * kN, primes[prime], t, g, L);
+        fwd_b_tile<false, false>(a, twb_all + (size_t)prime * kN, primes[prime], t, g, L);
         __syncthreads();
     }
 }
@@ -1117,7 +1185,7 @@ __global__ __launch_bounds__(kTileThreads* kFusedGroups) void k_ntt_inv_fused(ui
     uint64_t* L = lds + grp * kLdsWords;
     const uint64_t* in = job_src(js, blockIdx.x, data, off);
     for (int t = grp; t < 16; t += kFusedGroups) {
-        inv_b_tile<false, false>(a, in, JobIn{nullptr, nullptr}, P, twb_all + (size_t)prime * kN, t, g, L);
+        inv_b_tile<false, false, false>(a, in, JobIn{nullptr, nullptr}, P, twb_all + (size_t)prime * kN, t, g, L);
         __syncthreads();
     }
     for (int t = grp; t < 16; t += kFusedGroups) {
@@ -1150,6 +1218,10 @@ hipError_t launch_ntt(const Context& ctx, uint64_t* data, const JobSpec& js_in, 
             if (js.src2 && ctx.moduli[js.pmap[i]] >= (1ull << 60)) return hipErrorInvalidValue;
         mode = NttMode::TwoPass;
     }
+    if (js.scale) {
+        if (!inverse) return hipErrorInvalidValue;
+        mode = NttMode::TwoPass;
+    }
     if (js.lift) {
         // a lifted input: dense forward specs, two-pass kernels only
         if (js.jobs || inverse) return hipErrorInvalidValue;
@@ -1170,6 +1242,17 @@ hipError_t launch_ntt(const Context& ctx, uint64_t* data, const JobSpec& js_in, 
     return err;
 }
 
+hipError_t launch_ntt_fwd_b(const Context& ctx, uint64_t* data, const JobSpec& js, uint32_t n_jobs, hipStream_t st) {
+    if (n_jobs == 0) return hipSuccess;
+    const uint32_t n_primes = js.jobs ? js.n_primes : js.period;
+    const int pi = prof_begin(ctx, "ntt_fwd_2pass", (double)n_jobs * 2 * kN * 8 + (double)n_primes * kN * sizeof(TwPair), st);
+    hipLaunchKernelGGL(k_ntt_fwd_b<true>, dim3(16, n_jobs), dim3(kTileThreads), 0, st, data, js, ctx.d_twb, ctx.d_primes);
+    prof_end(ctx, pi, st);
+    return hipGetLastError();
+}
+
+// a_done (the launchers that end in a combine): the buffer already holds the first pass's output as the basis conversion
+// leaves it (bconv_ntt.hip: tiles of 16 blocks column-major); the second pass alone is launched.
 // launch_ntt_inv_ks for a key-switch list of n items (item c: extension ext[c] [D][E][N], key evk[c])
 hipError_t launch_ntt_inv_ksl(const Context& ctx, uint64_t* acc, const JobSpec& js, uint32_t n_jobs,
                               const uint64_t* const* ext, const uint64_t* const* evk, uint32_t n, uint32_t D,
@@ -1191,13 +1274,13 @@ hipError_t launch_ntt_inv_ksl(const Context& ctx, uint64_t* acc, const JobSpec& 
                          (double)js.n_primes * kN * sizeof(TwPair);
     const int pi = prof_begin(ctx, "ntt_inv_ks", bytes, st);
     const dim3 grid(16, n_jobs), block(kTileThreads);
-    switch (D) {
-        case 1: hipLaunchKernelGGL(k_ntt_inv_b_ksl<1>, grid, block, 0, st, acc, js, ctx.d_itwb, ctx.d_primes, ka); break;
-        case 2: hipLaunchKernelGGL(k_ntt_inv_b_ksl<2>, grid, block, 0, st, acc, js, ctx.d_itwb, ctx.d_primes, ka); break;
-        case 3: hipLaunchKernelGGL(k_ntt_inv_b_ksl<3>, grid, block, 0, st, acc, js, ctx.d_itwb, ctx.d_primes, ka); break;
-        default: hipLaunchKernelGGL(k_ntt_inv_b_ksl<4>, grid, block, 0, st, acc, js, ctx.d_itwb, ctx.d_primes, ka); break;
-    }
-    hipLaunchKernelGGL(k_ntt_inv_a, grid, block, 0, st, acc, js, ctx.d_itw, ctx.d_primes);
+    const bool cm = js.scale != nullptr;
+    auto k = D == 1   ? (cm ? k_ntt_inv_b_ksl<1, true> : k_ntt_inv_b_ksl<1, false>)
+             : D == 2 ? (cm ? k_ntt_inv_b_ksl<2, true> : k_ntt_inv_b_ksl<2, false>)
+             : D == 3 ? (cm ? k_ntt_inv_b_ksl<3, true> : k_ntt_inv_b_ksl<3, false>)
+                      : (cm ? k_ntt_inv_b_ksl<4, true> : k_ntt_inv_b_ksl<4, false>);
+    hipLaunchKernelGGL(k, grid, block, 0, st, acc, js, ctx.d_itwb, ctx.d_primes, ka);
+    hipLaunchKernelGGL(cm ? k_ntt_inv_a<true> : k_ntt_inv_a<false>, grid, block, 0, st, acc, js, ctx.d_itw, ctx.d_primes);
     prof_end(ctx, pi, st);
     return hipGetLastError();
 }
@@ -1210,7 +1293,7 @@ hipError_t launch_ntt_inv_ksl(const Context& ctx, uint64_t* acc, const JobSpec& 
 // k_ks_sub_list).
 hipError_t launch_ntt_fwd_ksl(const Context& ctx, uint64_t* y, const uint64_t* const* ext, const uint64_t* const* evk,
                               const uint64_t* add, uint64_t add_stride, uint32_t add_group, uint64_t* out, uint32_t n,
-                              uint32_t l, hipStream_t st, const uint32_t* gidx) {
+                              uint32_t l, hipStream_t st, const uint32_t* gidx, bool a_done) {
     const uint32_t D = (l + ctx.alpha - 1) / ctx.alpha, E = l + ctx.K;
     if (l == 0 || l > kMaxPmap || n == 0 || n > (uint32_t)kMaxList || D < 1 || D > 4 || add_group == 0)
         return hipErrorInvalidValue;
@@ -1249,17 +1332,17 @@ hipError_t launch_ntt_fwd_ksl(const Context& ctx, uint64_t* y, const uint64_t* c
     const uint32_t n_jobs = 2 * n * l;
     // algorithmic bytes: y read and written by pass A, read by pass B; ext limbs once per distinct ext, the keys and
     // out per item, addend polys once per group; tables
-    const double limbs = (double)n_jobs * 3 + ((double)distinct_ext * D + (double)n * (2.0 * D + 2) +
+    const double limbs = (double)n_jobs * (a_done ? 1 : 3) + ((double)distinct_ext * D + (double)n * (2.0 * D + 2) +
                                                (add ? (double)(n + add_group - 1) / add_group : 0.0)) * l;
     const int pi = prof_begin(ctx, "ntt_fwd_ksl", limbs * kN * 8 + (double)l * kN * sizeof(TwPair), st);
-    hipLaunchKernelGGL(k_ntt_fwd_a, dim3(16, n_jobs), dim3(kTileThreads), 0, st, y, js, ctx.d_tw, ctx.d_primes);
+    if (!a_done)
+        hipLaunchKernelGGL(k_ntt_fwd_a, dim3(16, n_jobs), dim3(kTileThreads), 0, st, y, js, ctx.d_tw, ctx.d_primes);
     const dim3 grid(16, n * l), block(2 * kTileThreads);
-    switch (D) {
-        case 1: hipLaunchKernelGGL(k_ntt_fwd_b_ksl<1>, grid, block, 0, st, y, ctx.d_twb, ctx.d_primes, f); break;
-        case 2: hipLaunchKernelGGL(k_ntt_fwd_b_ksl<2>, grid, block, 0, st, y, ctx.d_twb, ctx.d_primes, f); break;
-        case 3: hipLaunchKernelGGL(k_ntt_fwd_b_ksl<3>, grid, block, 0, st, y, ctx.d_twb, ctx.d_primes, f); break;
-        default: hipLaunchKernelGGL(k_ntt_fwd_b_ksl<4>, grid, block, 0, st, y, ctx.d_twb, ctx.d_primes, f); break;
-    }
+    auto k = D == 1   ? (a_done ? k_ntt_fwd_b_ksl<1, true> : k_ntt_fwd_b_ksl<1, false>)
+             : D == 2 ? (a_done ? k_ntt_fwd_b_ksl<2, true> : k_ntt_fwd_b_ksl<2, false>)
+             : D == 3 ? (a_done ? k_ntt_fwd_b_ksl<3, true> : k_ntt_fwd_b_ksl<3, false>)
+                      : (a_done ? k_ntt_fwd_b_ksl<4, true> : k_ntt_fwd_b_ksl<4, false>);
+    hipLaunchKernelGGL(k, grid, block, 0, st, y, ctx.d_twb, ctx.d_primes, f);
     prof_end(ctx, pi, st);
     return hipGetLastError();
 }
@@ -1277,13 +1360,13 @@ hipError_t launch_ntt_inv_ks(const Context& ctx, uint64_t* acc, const JobSpec& j
     const double bytes = ((double)n_jobs * (D + 3.0) + key_limbs) * kN * 8 + (double)js.n_primes * kN * sizeof(TwPair);
     const int pi = prof_begin(ctx, "ntt_inv_ks", bytes, st);
     const dim3 grid(16, n_jobs), block(kTileThreads);
-    switch (D) {
-        case 1: hipLaunchKernelGGL(k_ntt_inv_b_ks<1>, grid, block, 0, st, acc, js, ctx.d_itwb, ctx.d_primes, ka); break;
-        case 2: hipLaunchKernelGGL(k_ntt_inv_b_ks<2>, grid, block, 0, st, acc, js, ctx.d_itwb, ctx.d_primes, ka); break;
-        case 3: hipLaunchKernelGGL(k_ntt_inv_b_ks<3>, grid, block, 0, st, acc, js, ctx.d_itwb, ctx.d_primes, ka); break;
-        default: hipLaunchKernelGGL(k_ntt_inv_b_ks<4>, grid, block, 0, st, acc, js, ctx.d_itwb, ctx.d_primes, ka); break;
-    }
-    hipLaunchKernelGGL(k_ntt_inv_a, grid, block, 0, st, acc, js, ctx.d_itw, ctx.d_primes);
+    const bool cm = js.scale != nullptr;
+    auto k = D == 1   ? (cm ? k_ntt_inv_b_ks<1, true> : k_ntt_inv_b_ks<1, false>)
+             : D == 2 ? (cm ? k_ntt_inv_b_ks<2, true> : k_ntt_inv_b_ks<2, false>)
+             : D == 3 ? (cm ? k_ntt_inv_b_ks<3, true> : k_ntt_inv_b_ks<3, false>)
+                      : (cm ? k_ntt_inv_b_ks<4, true> : k_ntt_inv_b_ks<4, false>);
+    hipLaunchKernelGGL(k, grid, block, 0, st, acc, js, ctx.d_itwb, ctx.d_primes, ka);
+    hipLaunchKernelGGL(cm ? k_ntt_inv_a<true> : k_ntt_inv_a<false>, grid, block, 0, st, acc, js, ctx.d_itw, ctx.d_primes);
     prof_end(ctx, pi, st);
     return hipGetLastError();
 }
@@ -1344,12 +1427,13 @@ hipError_t launch_ntt_fwd_lsub(const Context& ctx, uint64_t* y, uint32_t n_terms
 // Forward NTT of a ModDown's converted P part y [n_polys][l][N] (coefficients, limb i over prime i; dense) whose pass
 // B ends in k_sub_scale's combine: out[pc][i] = (x[pc][i] - NTT(y)[pc][i]) s_i (+ the addend).  y is left holding
 // the first pass's intermediate.  Same argument meaning as launch_sub_scale.  lift (optional): y's input is instead
-// formed by the first pass from one limb per poly (JobSpec.lift).
+// formed by the first pass from one limb per poly (JobSpec.lift).  With a_done, y comes times s_i.
 hipError_t launch_ntt_fwd_sub(const Context& ctx, uint64_t* y, const uint64_t* x, uint64_t x_pstride,
                               const uint64_t* add, uint64_t add_pstride, uint32_t add_div, uint32_t add_group,
                               uint64_t* out, uint64_t out_pstride, uint32_t n_polys, uint32_t l, const TwPair* s,
-                              hipStream_t st, const uint64_t* lift, uint64_t lift_pstride, uint64_t lift_q) {
-    if (l == 0 || l > kMaxPmap || n_polys == 0) return hipErrorInvalidValue;
+                              hipStream_t st, const uint64_t* lift, uint64_t lift_pstride, uint64_t lift_q,
+                              bool a_done) {
+    if (l == 0 || l > kMaxPmap || n_polys == 0 || (a_done && lift)) return hipErrorInvalidValue;
     JobSpec js{};
     js.n_polys = n_polys;
     js.period = l;
@@ -1371,12 +1455,13 @@ hipError_t launch_ntt_fwd_sub(const Context& ctx, uint64_t* y, const uint64_t* x
     // algorithmic bytes: y read (or the lift source, once per poly) and written by pass A, read by pass B; x read,
     // out written; the addends; tables
     const double n_add = add ? (double)n_polys / ca.add_div : 0.0;
-    const double reads_a = lift ? (double)n_polys : (double)n_jobs;
+    const double reads_a = a_done ? -(double)n_jobs : lift ? (double)n_polys : (double)n_jobs;
     const double bytes = ((double)n_jobs * 4 + reads_a + n_add * l) * kN * 8 + (double)l * kN * sizeof(TwPair);
     const int pi = prof_begin(ctx, "ntt_fwd_sub", bytes, st);
     const dim3 grid(16, n_jobs), block(kTileThreads);
-    hipLaunchKernelGGL(k_ntt_fwd_a, grid, block, 0, st, y, js, ctx.d_tw, ctx.d_primes);
-    hipLaunchKernelGGL(k_ntt_fwd_b_sub, grid, block, 0, st, y, js, ctx.d_twb, ctx.d_primes, ca, x, add, out);
+    if (!a_done) hipLaunchKernelGGL(k_ntt_fwd_a, grid, block, 0, st, y, js, ctx.d_tw, ctx.d_primes);
+    auto k = a_done ? k_ntt_fwd_b_sub<true> : k_ntt_fwd_b_sub<false>;
+    hipLaunchKernelGGL(k, grid, block, 0, st, y, js, ctx.d_twb, ctx.d_primes, ca, x, add, out);
     prof_end(ctx, pi, st);
     return hipGetLastError();
 }
@@ -1391,7 +1476,7 @@ hipError_t launch_ntt_fwd_sub(const Context& ctx, uint64_t* y, const uint64_t* x
 hipError_t launch_ntt_fwd_mdr(const Context& ctx, uint64_t* T, uint32_t B, uint32_t l, const uint64_t* ext,
                               const uint64_t* evk, const uint64_t* ta, const uint64_t* tb, const uint64_t* add,
                               uint64_t add_pstride, uint64_t* out, const TwPair* pmod, const TwPair* cfin,
-                              hipStream_t st, const int64_t* post, bool own_from_inputs) {
+                              hipStream_t st, const int64_t* post, bool own_from_inputs, bool a_done) {
     const uint32_t D = (l + ctx.alpha - 1) / ctx.alpha, E = l + ctx.K;
     if (l < 2 || l > kMaxPmap || B == 0 || D < 1 || D > 4 || (ta && (!tb || add)) || (!ta && !add) ||
         own_from_inputs != (ta != nullptr) || ctx.alpha == 0)
@@ -1426,17 +1511,16 @@ hipError_t launch_ntt_fwd_mdr(const Context& ctx, uint64_t* T, uint32_t B, uint3
     // when the own digit's word is formed from the inputs), the 4 product inputs or 2 addend limbs, 2 outputs; the
     // level's evk limbs and the twiddle tables once
     const double n_ext = own_from_inputs ? D - 1.0 : (double)D;
-    const double limbs = (double)n_jobs * 3 + (double)B * (l - 1) * (n_ext + (ta ? 4 : add ? 2 : 0) + 2) +
+    const double limbs = (double)n_jobs * (a_done ? 1 : 3) + (double)B * (l - 1) * (n_ext + (ta ? 4 : add ? 2 : 0) + 2) +
                          2.0 * D * (l - 1);
     const int pi = prof_begin(ctx, "ntt_fwd_mdr", limbs * kN * 8 + (double)(l - 1) * kN * sizeof(TwPair), st);
-    hipLaunchKernelGGL(k_ntt_fwd_a, dim3(16, n_jobs), dim3(kTileThreads), 0, st, T, js, ctx.d_tw, ctx.d_primes);
+    if (!a_done)
+        hipLaunchKernelGGL(k_ntt_fwd_a, dim3(16, n_jobs), dim3(kTileThreads), 0, st, T, js, ctx.d_tw, ctx.d_primes);
     const dim3 grid(16, B * (l - 1)), block(2 * kTileThreads);
-    switch (D) {
-        case 1: launch_b_mdr<1>(grid, block, st, T, ctx.d_twb, ctx.d_primes, f); break;
-        case 2: launch_b_mdr<2>(grid, block, st, T, ctx.d_twb, ctx.d_primes, f); break;
-        case 3: launch_b_mdr<3>(grid, block, st, T, ctx.d_twb, ctx.d_primes, f); break;
-        default: launch_b_mdr<4>(grid, block, st, T, ctx.d_twb, ctx.d_primes, f); break;
-    }
+    if (a_done)
+        launch_b_mdr_d<true>(D, grid, block, st, T, ctx.d_twb, ctx.d_primes, f);
+    else
+        launch_b_mdr_d<false>(D, grid, block, st, T, ctx.d_twb, ctx.d_primes, f);
     prof_end(ctx, pi, st);
     return hipGetLastError();
 }
@@ -1455,11 +1539,12 @@ hipError_t launch_ntt_kernels(const Context& ctx, uint64_t* data, const JobSpec&
     // pass B reads pass B's table (the same pairs, its last four stages' entries reordered per block)
     const dim3 grid(16, n_jobs), block(kTileThreads);
     if (inverse) {
-        hipLaunchKernelGGL(k_ntt_inv_b, grid, block, 0, st, data, js, twb, ctx.d_primes);
-        hipLaunchKernelGGL(k_ntt_inv_a, grid, block, 0, st, data, js, tw, ctx.d_primes);
+        const bool cm = js.scale != nullptr;
+        hipLaunchKernelGGL(cm ? k_ntt_inv_b<true> : k_ntt_inv_b<false>, grid, block, 0, st, data, js, twb, ctx.d_primes);
+        hipLaunchKernelGGL(cm ? k_ntt_inv_a<true> : k_ntt_inv_a<false>, grid, block, 0, st, data, js, tw, ctx.d_primes);
     } else {
         hipLaunchKernelGGL(k_ntt_fwd_a, grid, block, 0, st, data, js, tw, ctx.d_primes);
-        hipLaunchKernelGGL(k_ntt_fwd_b, grid, block, 0, st, data, js, twb, ctx.d_primes);
+        hipLaunchKernelGGL(k_ntt_fwd_b<false>, grid, block, 0, st, data, js, twb, ctx.d_primes);
     }
     return hipGetLastError();
 }

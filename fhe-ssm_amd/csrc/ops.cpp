@@ -16,6 +16,7 @@
 #include <stdexcept>
 #include <string>
 
+#include "bconv_ntt.hpp"
 #include "engine.hpp"
 #include "ops.hpp"
 
@@ -45,7 +46,7 @@ hipError_t launch_mdr_combine_ks(const Context& ctx, const uint64_t* ext, const 
                                  const uint64_t* ta = nullptr, const uint64_t* tb = nullptr);
 hipError_t launch_ntt_fwd_ksl(const Context& ctx, uint64_t* y, const uint64_t* const* ext, const uint64_t* const* evk,
                               const uint64_t* add, uint64_t add_stride, uint32_t add_group, uint64_t* out, uint32_t n,
-                              uint32_t l, hipStream_t st, const uint32_t* gidx = nullptr);
+                              uint32_t l, hipStream_t st, const uint32_t* gidx = nullptr, bool a_done = false);
 hipError_t launch_ntt_inv_ksl(const Context& ctx, uint64_t* acc, const JobSpec& js, uint32_t n_jobs,
                               const uint64_t* const* ext, const uint64_t* const* evk, uint32_t n, uint32_t D,
                               uint32_t E, hipStream_t st);
@@ -55,7 +56,7 @@ hipError_t launch_ntt_fwd_sub(const Context& ctx, uint64_t* y, const uint64_t* x
                               const uint64_t* add, uint64_t add_pstride, uint32_t add_div, uint32_t add_group,
                               uint64_t* out, uint64_t out_pstride, uint32_t n_polys, uint32_t l, const TwPair* s,
                               hipStream_t st, const uint64_t* lift = nullptr, uint64_t lift_pstride = 0,
-                              uint64_t lift_q = 0);
+                              uint64_t lift_q = 0, bool a_done = false);
 hipError_t launch_ntt_fwd_lsub(const Context& ctx, uint64_t* y, uint32_t n_terms, const uint64_t* const* x,
                                const uint32_t* stride, const uint64_t* C, const uint64_t* add, uint64_t* out,
                                uint64_t out_pstride, uint32_t n_polys, uint32_t l, const TwPair* s, hipStream_t st,
@@ -63,7 +64,8 @@ hipError_t launch_ntt_fwd_lsub(const Context& ctx, uint64_t* y, uint32_t n_terms
 hipError_t launch_ntt_fwd_mdr(const Context& ctx, uint64_t* T, uint32_t B, uint32_t l, const uint64_t* ext,
                               const uint64_t* evk, const uint64_t* ta, const uint64_t* tb, const uint64_t* add,
                               uint64_t add_pstride, uint64_t* out, const TwPair* pmod, const TwPair* cfin,
-                              hipStream_t st, const int64_t* post = nullptr, bool own_from_inputs = false);
+                              hipStream_t st, const int64_t* post = nullptr, bool own_from_inputs = false,
+                              bool a_done = false);
 hipError_t launch_sub_scale(const Context& ctx, const uint64_t* x, uint64_t x_pstride, const uint64_t* y,
                             uint64_t y_pstride, const uint64_t* add, uint64_t add_pstride, uint32_t add_div,
                             uint64_t* out, uint64_t out_pstride, uint32_t n_polys, uint32_t l, const TwPair* s,
@@ -389,12 +391,210 @@ static void check_level(const Context& ctx, uint32_t l) {
     if (num_digits(ctx, l) > 8) throw std::invalid_argument("more than 8 digits");
 }
 
+// ------------------------------------------------------------------ matrix-core conversions
+// Taken under the two-pass NTT for every chain whose primes have at least 35 bits (the reduction's quotient unit) and
+// conversions within the tables' limits; otherwise k_bconv and a whole forward NTT.
+enum MfKind : uint32_t { kMfModUp = 0, kMfDown = 1, kMfDownRescale = 2 };
+
+static bool mf_modup(const Context& ctx, uint32_t l) {
+    return ctx.ntt_mode == NttMode::TwoPass && ctx.mf_primes && ctx.alpha <= (uint32_t)kMfMaxIn &&
+           l + ctx.K <= kMfMaxOut;
+}
+static bool mf_moddown(const Context& ctx, uint32_t l) {
+    return ctx.ntt_mode == NttMode::TwoPass && ctx.mf_primes && ctx.K <= (uint32_t)kMfMaxIn && l <= kMfMaxOut;
+}
+
+// prod of the primes idx but idx[skip], mod q
+static uint64_t prod_mod(const Context& ctx, const std::vector<uint32_t>& idx, size_t skip, uint64_t q) {
+    uint64_t m = 1 % q;
+    for (size_t k = 0; k < idx.size(); k++)
+        if (k != skip) m = mulmod_h(m, ctx.moduli[idx[k]] % q, q);
+    return m;
+}
+
+static void mf_put(std::vector<uint64_t>& host, size_t at, const void* src, size_t bytes) {
+    if (host.size() < at + (bytes + 7) / 8) host.resize(at + (bytes + 7) / 8);
+    std::memcpy(host.data() + at, src, bytes);
+}
+
+// appends one conversion (sources in_idx, outputs out_idx at limb out_limb[j]) to a plan: the scale entries of its
+// sources, its slots and constants qhat_i col_scale_j
+static void mf_add(const Context& ctx, MfPlan& p, const std::vector<uint32_t>& in_idx,
+                   const std::vector<uint32_t>& out_idx, const std::vector<uint32_t>& out_limb, uint64_t in_off,
+                   uint64_t out_off, const std::vector<uint64_t>& col_scale) {
+    MfConv c{};
+    c.n_in = (uint32_t)in_idx.size();
+    c.n_out = (uint32_t)out_idx.size();
+    c.n_grp = (c.n_out + 3) / 4;
+    c.in_off = in_off;
+    c.out_off = out_off;
+    for (uint32_t i = 0; i < c.n_in; i++) {
+        const uint64_t q = ctx.moduli[in_idx[i]];
+        const PrimeInfo& pr = ctx.primes[in_idx[i]];
+        const uint64_t f = invmod_h(prod_mod(ctx, in_idx, i, q), q);
+        const uint64_t a = mulmod_h(pr.ninv, f, q), b = mulmod_h(pr.w1ninv, f, q);
+        const InvScale sc{TwPair{a, shoup_companion(a, q)}, TwPair{b, shoup_companion(b, q)}, 1};
+        mf_put(p.host, (size_t)in_idx[i] * (sizeof(InvScale) / 8), &sc, sizeof(sc));
+    }
+    std::vector<MfSlot> slots(4 * (size_t)c.n_grp);
+    for (uint32_t g = 0; g < c.n_grp; g++) {
+        bool open = true;
+        for (uint32_t j = 4 * g; j < std::min(4 * g + 4, c.n_out); j++) open = open && ctx.moduli[out_idx[j]] < (1ull << 56);
+        for (uint32_t j = 4 * g; j < 4 * g + 4; j++) {
+            const uint32_t jj = j < c.n_out ? j : 4 * g;
+            const uint64_t q = ctx.moduli[out_idx[jj]], nq = 0 - q;
+            const uint32_t bits = 64 - (uint32_t)__builtin_clzll(q);
+            MfSlot& s = slots[j];
+            s.q = q;
+            s.nq_lo = (int32_t)(uint32_t)nq;
+            s.nq_hi = (int32_t)(uint32_t)((nq - (uint64_t)(int64_t)s.nq_lo) >> 32);
+            s.sh = bits > 47 ? bits - 47 : 0;
+            s.M = (int32_t)(((unsigned __int128)1 << (64 + s.sh)) / q);
+            s.prime = out_idx[jj];
+            s.off = out_limb[jj];
+            s.flags = j < c.n_out ? 0 : kMfNone;
+        }
+        c.open |= (open ? 1u : 0u) << g;
+    }
+    c.slots_at = p.host.size();
+    mf_put(p.host, c.slots_at, slots.data(), slots.size() * sizeof(MfSlot));
+    std::vector<uint64_t> cm((size_t)c.n_in * c.n_out);
+    for (uint32_t j = 0; j < c.n_out; j++) {
+        const uint64_t q = ctx.moduli[out_idx[j]];
+        for (uint32_t i = 0; i < c.n_in; i++) {
+            const uint64_t m = prod_mod(ctx, in_idx, i, q);
+            cm[(size_t)i * c.n_out + j] = col_scale.empty() ? m : mulmod_h(m, col_scale[j], q);
+        }
+    }
+    c.cmat_at = p.host.size();
+    mf_put(p.host, c.cmat_at, cm.data(), cm.size() * 8);
+    p.ks = std::max(p.ks, (c.n_in + 7) / 8);
+    p.n_grp += c.n_grp;
+    p.conv.push_back(c);
+}
+
+static MfPlan mf_build(const Context& ctx, uint32_t kind, uint32_t l) {
+    MfPlan p;
+    p.host.assign((size_t)(ctx.L + ctx.K) * (sizeof(InvScale) / 8), 0);  // the scale table, zero: no factor
+    if (kind == kMfModUp) {
+        const uint32_t D = (l + ctx.alpha - 1) / ctx.alpha, E = l + ctx.K;
+        for (uint32_t d = 0; d < D; d++) {
+            const uint32_t lo = d * ctx.alpha, hi = std::min(lo + ctx.alpha, l);
+            std::vector<uint32_t> in_idx, out_idx, out_limb;
+            for (uint32_t i = lo; i < hi; i++) in_idx.push_back(i);
+            for (uint32_t t = 0; t < E; t++) {
+                if (t >= lo && t < hi) continue;
+                out_idx.push_back(t < l ? t : ctx.L + (t - l));
+                out_limb.push_back(t);
+            }
+            if (!out_idx.empty())
+                mf_add(ctx, p, in_idx, out_idx, out_limb, (uint64_t)lo * W, (uint64_t)d * E * W, {});
+        }
+    } else {
+        // the P limbs (l..E-1 of an extended poly) to the Q limbs, P^-1 folded into the columns
+        const bool rescale = kind == kMfDownRescale;
+        std::vector<uint32_t> in_idx, out_idx;
+        std::vector<uint64_t> col;
+        for (uint32_t k = 0; k < ctx.K; k++) in_idx.push_back(ctx.L + k);
+        for (uint32_t i = 0; i < (rescale ? l - 1 : l); i++) {
+            const uint64_t q = ctx.moduli[i];
+            out_idx.push_back(i);
+            col.push_back(invmod_h(prod_mod(ctx, in_idx, in_idx.size(), q), q));
+        }
+        if (rescale) {  // the dropped limb, a plain residue in the same order
+            const InvScale sc{TwPair{0, 0}, TwPair{0, 0}, 2};
+            mf_put(p.host, (size_t)(l - 1) * (sizeof(InvScale) / 8), &sc, sizeof(sc));
+        }
+        mf_add(ctx, p, in_idx, out_idx, out_idx, (uint64_t)l * W, 0, col);
+    }
+    p.words = (p.host.size() + 1) & ~(size_t)1;  // the operands are read 16 bytes at a time
+    for (auto& c : p.conv) {
+        c.tab_at = p.words;
+        p.words += (size_t)c.n_grp * p.ks * 2 * 64 * 2;
+    }
+    return p;
+}
+
+// the plan of a kind at a level, and its device copy: built once per context, or for an allocation-free call in its arena
+struct MfRef {
+    const MfPlan* plan;
+    uint64_t* dev;
+    const InvScale* scale() const { return (const InvScale*)dev; }
+};
+
+static MfRef mf_plan(Context& ctx, uint32_t kind, uint32_t l, hipStream_t st) {
+    const uint32_t key = kind | (l << 2);
+    auto it = ctx.mf_cache.find(key);
+    if (it == ctx.mf_cache.end()) it = ctx.mf_cache.emplace(key, mf_build(ctx, kind, l)).first;
+    MfPlan& p = it->second;
+    if (p.dev) return MfRef{&p, p.dev};
+    uint64_t* dev = nullptr;
+    if (ctx.arena) {
+        auto have = ctx.arena->mf.find(key);
+        if (have != ctx.arena->mf.end()) return MfRef{&p, have->second};
+        dev = (uint64_t*)arena_take(*ctx.arena, p.words * 8);
+        HIPX(arena_put(dev, p.host.data(), p.host.size() * 8, st));
+        ctx.arena->mf.emplace(key, dev);
+    } else {
+        HIPX(hipMalloc(&dev, p.words * 8));
+        const hipError_t e = hipMemcpy(dev, p.host.data(), p.host.size() * 8, hipMemcpyHostToDevice);
+        if (e != hipSuccess) {
+            (void)hipFree(dev);
+            HIPX(e);
+        }
+    }
+    for (const auto& c : p.conv) {
+        const hipError_t e = launch_mf_table(ctx, dev + c.cmat_at, (const MfSlot*)(dev + c.slots_at), dev + c.tab_at,
+                                             c.n_in, c.n_out, c.n_grp, p.ks, st);
+        if (e != hipSuccess) {
+            if (!ctx.arena) (void)hipFree(dev);
+            HIPX(e);
+        }
+    }
+    if (!ctx.arena) {
+        // later calls may come on other streams: the table is complete before the plan is kept
+        const hipError_t e = hipStreamSynchronize(st);
+        if (e != hipSuccess) {
+            (void)hipFree(dev);
+            HIPX(e);
+        }
+        p.dev = dev;
+    }
+    return MfRef{&p, dev};
+}
+
+// runs a plan's conversions and the first NTT pass of their outputs over B batch items; extra: the limb added to every
+// output (k_moddown_head), or null
+static void mf_convert(Context& ctx, const MfRef& r, const uint64_t* in, uint64_t in_bstride, const uint64_t* extra,
+                       uint64_t extra_bstride, uint64_t* out, uint64_t out_bstride, uint32_t B, hipStream_t st,
+                       const char* name = "bconv") {
+    MfArgs ma{};
+    ma.n_dig = (uint32_t)r.plan->conv.size();
+    ma.n_grp = r.plan->n_grp;
+    ma.in_bstride = in_bstride;
+    ma.out_bstride = out_bstride;
+    ma.extra_bstride = extra_bstride;
+    if (ma.n_dig == 0) return;
+    for (uint32_t d = 0; d < ma.n_dig; d++) {
+        const MfConv& c = r.plan->conv[d];
+        ma.dig[d] = MfDigit{(const MfSlot*)(r.dev + c.slots_at), r.dev + c.tab_at, c.in_off, c.out_off, c.n_in,
+                            c.n_out, c.n_grp, c.open};
+    }
+    HIPX(launch_bconv_ntt_a(ctx, r.plan->ks, in, extra, out, ma, B, name, st));
+}
+
 // ------------------------------------------------------------------ ModUp
-// x2c: [B][l][N] coefficient form (INTT already applied) of the polynomial to extend;
+// the factors the inverse NTT of a ModUp source folds into its last stage (null: plain coefficients)
+static const InvScale* modup_scale(Context& ctx, uint32_t l, hipStream_t st) {
+    return mf_modup(ctx, l) ? mf_plan(ctx, kMfModUp, l, st).scale() : nullptr;
+}
+
+// x2c: [B][l][N] inverse NTT (with modup_scale's factors) of the polynomial to extend;
 // ext: [B][D][E][N].  Fills every limb but the digits' own (neither read nor written here: the caller stores them in
 // evaluation form, or their consumer forms them).
 void modup_from_coef(Context& ctx, const uint64_t* x2c, uint64_t* ext, uint32_t B, uint32_t l, hipStream_t st) {
     const uint32_t D = num_digits(ctx, l), E = l + ctx.K, al = ctx.alpha;
+    const bool mf = mf_modup(ctx, l);
     std::vector<Job> jobs;
     for (uint32_t d = 0; d < D; d++) {
         const uint32_t lo = d * al, hi = std::min(lo + al, l);
@@ -408,15 +608,22 @@ void modup_from_coef(Context& ctx, const uint64_t* x2c, uint64_t* ext, uint32_t 
             out_idx.push_back(ext_prime(ctx, l, t));
             out_off.push_back(t);
         }
-        const BConvPlan& plan = bconv_plan(ctx, in_idx, out_idx);
-        HIPX(launch_bconv(ctx, plan, x2c, (uint64_t)l * W, in_off.data(), ext + (size_t)d * E * W,
-                          (uint64_t)D * E * W, out_off.data(), B, st));
+        if (!mf) {
+            const BConvPlan& plan = bconv_plan(ctx, in_idx, out_idx);
+            HIPX(launch_bconv(ctx, plan, x2c, (uint64_t)l * W, in_off.data(), ext + (size_t)d * E * W,
+                              (uint64_t)D * E * W, out_off.data(), B, st));
+        }
         for (uint32_t b = 0; b < B; b++)
             for (uint32_t j = 0; j < out_off.size(); j++)
                 jobs.push_back(Job{(b * D + d) * E + out_off[j], out_idx[j]});
     }
     const JobSpec js = cached_jobs(ctx, "modup:" + std::to_string(B) + ":" + std::to_string(l), std::move(jobs));
     const uint32_t n_jobs = B * D * (E) - B * l;  // every limb of every digit except the digit's own
+    if (mf) {
+        mf_convert(ctx, mf_plan(ctx, kMfModUp, l, st), x2c, (uint64_t)l * W, nullptr, 0, ext, (uint64_t)D * E * W, B, st);
+        HIPX(launch_ntt_fwd_b(ctx, ext, js, n_jobs, st));
+        return;
+    }
     HIPX(launch_ntt(ctx, ext, js, n_jobs, false, ctx.ntt_mode, st));
 }
 
@@ -440,6 +647,7 @@ void modup(Context& ctx, const uint64_t* x, uint64_t* ext, uint32_t B, uint32_t 
     js.copy_pstride = (uint64_t)D * E * W;
     js.copy_alpha = al;
     js.copy_E = E;
+    js.scale = modup_scale(ctx, l, st);
     HIPX(launch_ntt(ctx, xc, js, B * l, true, ctx.ntt_mode, st));
     modup_from_coef(ctx, xc, ext, B, l, st);
 }
@@ -449,6 +657,31 @@ void ks_inner(Context& ctx, const uint64_t* ext, const uint64_t* evk, uint64_t* 
               hipStream_t st) {
     check_level(ctx, l);
     HIPX(launch_ks_inner(ctx, ext, evk, acc, B, l, st));
+}
+
+// the limb added in a ModDown conversion (k_moddown_head) from the P limbs' digit words y: with the rescale, limb l-1 of
+// the polys (coefficients, at xlast) and of the addend (addc, or null) enter it
+static void moddown_head(Context& ctx, const uint64_t* y, uint64_t y_bstride, uint64_t* e, uint64_t e_bstride, uint32_t l,
+                         bool rescale, const uint64_t* xlast, uint64_t x_bstride, const uint64_t* addc, uint32_t n_polys,
+                         hipStream_t st) {
+    MfHeadArgs ha{};
+    ha.n_in = ctx.K;
+    ha.exact = ctx.moddown_exact ? 1 : 0;
+    ha.rescale = rescale ? 1 : 0;
+    ha.last = l - 1;
+    std::vector<uint32_t> in_idx;
+    for (uint32_t k = 0; k < ctx.K; k++) in_idx.push_back(ctx.L + k);
+    const uint64_t ql = ctx.moduli[l - 1];
+    for (uint32_t k = 0; k < ctx.K; k++) {
+        const unsigned __int128 c = (~(unsigned __int128)0) / ctx.moduli[ctx.L + k];  // floor(2^128 / p_k)
+        ha.fix[k][0] = (uint64_t)c;
+        ha.fix[k][1] = (uint64_t)(c >> 64);
+        ha.c[k] = prod_mod(ctx, in_idx, k, ql);
+    }
+    const uint64_t P = prod_mod(ctx, in_idx, in_idx.size(), ql);
+    ha.c[kMfMaxIn] = P ? ql - P : 0;
+    ha.pinv = pinv_tab(ctx)[l - 1];
+    HIPX(launch_moddown_head(ctx, y, y_bstride, e, e_bstride, xlast, x_bstride, addc, ha, n_polys, st));
 }
 
 // ------------------------------------------------------------------ ModDown
@@ -464,9 +697,25 @@ void moddown_inplace(Context& ctx, uint64_t* x, uint32_t n_polys, uint32_t l, co
     std::vector<Job> jobs;
     for (uint32_t pc = 0; pc < n_polys; pc++)
         for (uint32_t k = 0; k < K; k++) jobs.push_back(Job{pc * xs + l + k, ctx.L + k});
-    const JobSpec js = cached_jobs(ctx, "mdP:" + std::to_string(n_polys) + ":" + std::to_string(l) + ":" +
-                                            std::to_string(xs),
-                                   std::move(jobs));
+    JobSpec js = cached_jobs(ctx, "mdP:" + std::to_string(n_polys) + ":" + std::to_string(l) + ":" +
+                                      std::to_string(xs),
+                             std::move(jobs));
+    uint64_t* conv = (uint64_t*)ws_get(ctx, WS_CONV, (size_t)n_polys * l * W * 8);
+    const uint64_t aps = add_pstride < 0 ? (uint64_t)add_div * l * W : (uint64_t)add_pstride;
+    if (mf_moddown(ctx, l)) {
+        const MfRef r = mf_plan(ctx, kMfDown, l, st);
+        js.scale = r.scale();
+        HIPX(launch_ntt(ctx, x, js, n_polys * K, true, ctx.ntt_mode, st));
+        uint64_t* e = nullptr;
+        if (ctx.moddown_exact) {
+            e = (uint64_t*)ws_get(ctx, WS_LAST, (size_t)n_polys * W * 8);
+            moddown_head(ctx, x + (size_t)l * W, (uint64_t)xs * W, e, W, l, false, nullptr, 0, nullptr, n_polys, st);
+        }
+        mf_convert(ctx, r, x, (uint64_t)xs * W, e, W, conv, (uint64_t)l * W, n_polys, st);
+        HIPX(launch_ntt_fwd_sub(ctx, conv, x, (uint64_t)xs * W, add, aps, add_div, add_group, out, (uint64_t)l * W,
+                                n_polys, l, pinv_tab(ctx).data(), st, nullptr, 0, 0, true));
+        return;
+    }
     HIPX(launch_ntt(ctx, x, js, n_polys * K, true, ctx.ntt_mode, st));
     std::vector<uint32_t> in_idx, in_off, out_idx, out_off;
     for (uint32_t k = 0; k < K; k++) {
@@ -478,11 +727,9 @@ void moddown_inplace(Context& ctx, uint64_t* x, uint32_t n_polys, uint32_t l, co
         out_off.push_back(i);
     }
     const BConvPlan& plan = bconv_plan(ctx, in_idx, out_idx, ctx.moddown_exact);
-    uint64_t* conv = (uint64_t*)ws_get(ctx, WS_CONV, (size_t)n_polys * l * W * 8);
     HIPX(launch_bconv(ctx, plan, x, (uint64_t)xs * W, in_off.data(), conv, (uint64_t)l * W, out_off.data(), n_polys,
                       st));
     const std::vector<TwPair> pinv(pinv_tab(ctx).begin(), pinv_tab(ctx).begin() + l);
-    const uint64_t aps = add_pstride < 0 ? (uint64_t)add_div * l * W : (uint64_t)add_pstride;
     if (ctx.ntt_mode == NttMode::TwoPass) {
         // the forward NTT of conv ends in the combine (conv is never stored in evaluation form)
         HIPX(launch_ntt_fwd_sub(ctx, conv, x, (uint64_t)xs * W, add, aps, add_div, add_group, out, (uint64_t)l * W,
@@ -516,7 +763,10 @@ void moddown_rescale(Context& ctx, uint64_t* x, uint32_t n_polys, uint32_t l, co
         jobs.push_back(Job{pc * E + l - 1, l - 1});
         for (uint32_t k = 0; k < K; k++) jobs.push_back(Job{pc * E + l + k, ctx.L + k});
     }
-    const JobSpec js = cached_jobs(ctx, "mdrP:" + std::to_string(n_polys) + ":" + std::to_string(l), std::move(jobs));
+    JobSpec js = cached_jobs(ctx, "mdrP:" + std::to_string(n_polys) + ":" + std::to_string(l), std::move(jobs));
+    const bool mf = mf_moddown(ctx, l);
+    const MfRef r = mf ? mf_plan(ctx, kMfDownRescale, l, st) : MfRef{nullptr, nullptr};
+    if (mf) js.scale = r.scale();
     if (x_from_ext)  // those limbs of x are the evk inner product, formed by the transform's first pass
         HIPX(launch_ntt_inv_ks(ctx, x, js, n_polys * (K + 1), ext, evk, num_digits(ctx, l), E, st));
     else
@@ -528,6 +778,7 @@ void moddown_rescale(Context& ctx, uint64_t* x, uint32_t n_polys, uint32_t l, co
         JobSpec ja = regular_jobs(n_polys, {l - 1});
         ja.src = add + (size_t)(l - 1) * W;
         ja.src_period = l;
+        if (mf) ja.scale = r.scale();
         HIPX(launch_ntt(ctx, addc, ja, n_polys, true, ctx.ntt_mode, st));
     }
     const std::vector<TwPair>& ptab = pinv_tab(ctx);
@@ -544,11 +795,18 @@ void moddown_rescale(Context& ctx, uint64_t* x, uint32_t n_polys, uint32_t l, co
         in_off.push_back(l + k);
     }
     for (uint32_t i = 0; i < l; i++) out_idx.push_back(i);
-    const BConvPlan& plan = bconv_plan(ctx, in_idx, out_idx, ctx.moddown_exact, col);
     uint64_t* T = (uint64_t*)ws_get(ctx, WS_RTMP, (size_t)n_polys * (l - 1) * W * 8);
     const uint64_t xps = (uint64_t)E * W;
-    HIPX(launch_bconv_mdr(ctx, plan, x, xps, in_off.data(), T, n_polys, x + (size_t)(l - 1) * W, xps, addc,
-                          pinv[l - 1], st));
+    if (mf) {
+        // the limb to add takes the place of limb l-1 of x
+        uint64_t* e = x + (size_t)(l - 1) * W;
+        moddown_head(ctx, x + (size_t)l * W, xps, e, xps, l, true, e, xps, addc, n_polys, st);
+        mf_convert(ctx, r, x, xps, e, xps, T, (uint64_t)(l - 1) * W, n_polys, st, "bconv_mdr");
+    } else {
+        const BConvPlan& plan = bconv_plan(ctx, in_idx, out_idx, ctx.moddown_exact, col);
+        HIPX(launch_bconv_mdr(ctx, plan, x, xps, in_off.data(), T, n_polys, x + (size_t)(l - 1) * W, xps, addc,
+                              pinv[l - 1], st));
+    }
     std::vector<uint32_t> pm(l - 1);
     for (uint32_t i = 0; i + 1 < l; i++) pm[i] = i;
     // a relinearization: T's forward NTT finishes with the combine in its second pass (the addend formed from the
@@ -565,10 +823,13 @@ void moddown_rescale(Context& ctx, uint64_t* x, uint32_t n_polys, uint32_t l, co
             cfin[i] = TwPair{v, shoup_companion(v, q)};
         }
         HIPX(launch_ntt_fwd_mdr(ctx, T, n_polys / 2, l, ext, evk, ta, tb, ta ? nullptr : add, (uint64_t)l * W, out,
-                                pmod_tab(ctx).data(), cfin.data(), st, aff ? &aff->post : nullptr, own_from_inputs));
+                                pmod_tab(ctx).data(), cfin.data(), st, aff ? &aff->post : nullptr, own_from_inputs, mf));
         return;
     }
-    HIPX(launch_ntt(ctx, T, regular_jobs(n_polys, pm), n_polys * (l - 1), false, ctx.ntt_mode, st));
+    if (mf)
+        HIPX(launch_ntt_fwd_b(ctx, T, regular_jobs(n_polys, pm), n_polys * (l - 1), st));
+    else
+        HIPX(launch_ntt(ctx, T, regular_jobs(n_polys, pm), n_polys * (l - 1), false, ctx.ntt_mode, st));
     if (ext && ta)  // the addend formed from the product's inputs (add holds limb l-1 only, read above)
         HIPX(launch_mdr_combine_ks(ctx, ext, evk, nullptr, 0, T, out, n_polys / 2, l, pinv.data(), qlinv.data(), st,
                                    ta, tb));
@@ -609,7 +870,10 @@ void ks_moddown_list(Context& ctx, const uint64_t* const* ext, const uint64_t* c
     std::vector<Job> jobs;
     for (uint32_t pc = 0; pc < 2 * n; pc++)
         for (uint32_t k = 0; k < K; k++) jobs.push_back(Job{pc * E + l + k, ctx.L + k});
-    const JobSpec js = cached_jobs(ctx, "mdP:" + std::to_string(2 * n) + ":" + std::to_string(l), std::move(jobs));
+    JobSpec js = cached_jobs(ctx, "mdP:" + std::to_string(2 * n) + ":" + std::to_string(l), std::move(jobs));
+    const bool mf = mf_moddown(ctx, l);
+    const MfRef r = mf ? mf_plan(ctx, kMfDown, l, st) : MfRef{nullptr, nullptr};
+    if (mf) js.scale = r.scale();
     if (fused) {
         // the P limbs' inner products are formed by their inverse NTT's first pass
         ctx.n_keyswitch += n;
@@ -629,10 +893,17 @@ void ks_moddown_list(Context& ctx, const uint64_t* const* ext, const uint64_t* c
         out_idx.push_back(i);
         col[i] = pinv[i].w;
     }
-    const BConvPlan& plan = bconv_plan(ctx, in_idx, out_idx, ctx.moddown_exact, col);
     uint64_t* conv = (uint64_t*)ws_get(ctx, WS_CONV, (size_t)2 * n * l * W * 8);
-    HIPX(launch_bconv(ctx, plan, acc, (uint64_t)E * W, in_off.data(), conv, (uint64_t)l * W, out_idx.data(), 2 * n,
-                      st));
+    if (mf) {
+        // the limb to add (exact form) in limb l-1 of the accumulator, whose Q limbs are never formed
+        uint64_t* e = ctx.moddown_exact ? acc + (size_t)(l - 1) * W : nullptr;
+        if (e) moddown_head(ctx, acc + (size_t)l * W, (uint64_t)E * W, e, (uint64_t)E * W, l, false, nullptr, 0, nullptr, 2 * n, st);
+        mf_convert(ctx, r, acc, (uint64_t)E * W, e, (uint64_t)E * W, conv, (uint64_t)l * W, 2 * n, st);
+    } else {
+        const BConvPlan& plan = bconv_plan(ctx, in_idx, out_idx, ctx.moddown_exact, col);
+        HIPX(launch_bconv(ctx, plan, acc, (uint64_t)E * W, in_off.data(), conv, (uint64_t)l * W, out_idx.data(), 2 * n,
+                          st));
+    }
     // the combine applies the automorphisms as it stores, unless out overlaps the addends' polys 0 (a permuted store
     // may land on words another workgroup has still to read): then the key switch goes to a workspace first
     const uint64_t* add_end = add ? add + (size_t)((n - 1) / std::max(add_group, 1u)) * add_stride + (size_t)l * W : nullptr;
@@ -641,9 +912,12 @@ void ks_moddown_list(Context& ctx, const uint64_t* const* ext, const uint64_t* c
     if (fused) {
         // the forward NTT of conv ends in the combine (conv never stored in evaluation form)
         HIPX(launch_ntt_fwd_ksl(ctx, conv, ext, evk, add, add_stride, add_group, ks, n, l, st,
-                                ks == out ? gidx : nullptr));
+                                ks == out ? gidx : nullptr, mf));
     } else {
-        HIPX(launch_ntt(ctx, conv, regular_jobs(2 * n, out_idx), 2 * n * l, false, ctx.ntt_mode, st));
+        if (mf)
+            HIPX(launch_ntt_fwd_b(ctx, conv, regular_jobs(2 * n, out_idx), 2 * n * l, st));
+        else
+            HIPX(launch_ntt(ctx, conv, regular_jobs(2 * n, out_idx), 2 * n * l, false, ctx.ntt_mode, st));
         HIPX(launch_ks_sub_list(ctx, ext, evk, conv, add, add_stride, add_group, ks, n, l, pinv.data(), st));
     }
     if (gidx && ks != out) HIPX(launch_automorph_list(ctx, ks, out, n, l, gidx, st));
@@ -750,7 +1024,11 @@ static void relin_tail(Context& ctx, uint64_t* d01, uint64_t* x2c, uint64_t* ext
     uint64_t* acc = (uint64_t*)ws_get(ctx, WS_ACC, (size_t)B * 2 * E * W * 8);
     std::vector<uint32_t> pm(l);
     for (uint32_t i = 0; i < l; i++) pm[i] = i;
-    if (!x2c_coef) HIPX(launch_ntt(ctx, x2c, regular_jobs(B, pm), B * l, true, ctx.ntt_mode, st));
+    if (!x2c_coef) {
+        JobSpec js = regular_jobs(B, pm);
+        js.scale = modup_scale(ctx, l, st);
+        HIPX(launch_ntt(ctx, x2c, js, B * l, true, ctx.ntt_mode, st));
+    }
     modup_from_coef(ctx, x2c, ext, B, l, st);
     if (!do_rescale) {
         HIPX(launch_ks_inner(ctx, ext, evk, acc, B, l, st));
@@ -801,6 +1079,7 @@ void hmult(Context& ctx, const uint64_t* a, const uint64_t* b, uint32_t B, uint3
     js.copy_alpha = ctx.alpha;
     js.copy_E = E;
     js.copy_from = own ? l - 1 : 0;
+    js.scale = modup_scale(ctx, l, st);
     HIPX(launch_ntt(ctx, x2c, js, B * l, true, ctx.ntt_mode, st));
     if (from_inputs)
         relin_tail(ctx, d01, x2c, ext, B, l, evk, out, true, st, a, b, true, aff, own);
