@@ -338,6 +338,7 @@ __device__ __forceinline__ void fwd_b_tile(uint64_t* __restrict__ a, const TwPai
 struct KsIn {
     const uint64_t* e;  // the job's evk limb of digit 0 (digit d at e + d es)
     size_t xs, es;      // digit strides of the extension (in) and of the key, in words
+    const uint64_t* add = nullptr;  // a limb added P-fold to the inner product (a Q limb's: P.pmod), or null
 };
 
 // kCm: the limb will end column-major within 16 rows (InvScale): this tile's 16 rows are stored in their own 4,096 words
@@ -355,25 +356,28 @@ __device__ __forceinline__ void inv_b_tile(uint64_t* a, const uint64_t* in, JobI
     uint64_t* L = lds + bl * 272;
     uint64_t x[16];
     if constexpr (kD > 0) {
-        // two words at a time, all their digit loads issued before the products (sums of kD <= 4 products of
+        // two words at a time, all their digit loads issued before the products (sums of kD + 1 <= 5 products of
         // residues below q < 2^60: the high word stays below q)
         const Barrett br{q, P.mu_hi, P.mu_lo};
         const uint64_t* e = ks.e + 256 * b;
 #pragma unroll
         for (int k0 = 0; k0 < 16; k0 += 2) {
-            uint64_t xv[2][kD], ev[2][kD];
+            uint64_t xv[2][kD], ev[2][kD], av[2] = {0, 0};
 #pragma unroll
-            for (int j = 0; j < 2; j++)
+            for (int j = 0; j < 2; j++) {
 #pragma unroll
                 for (int d = 0; d < kD; d++) {
                     xv[j][d] = src[d * ks.xs + rl + 16 * (k0 + j)];
                     ev[j][d] = e[d * ks.es + rl + 16 * (k0 + j)];
                 }
+                if (ks.add) av[j] = ks.add[256 * b + rl + 16 * (k0 + j)];
+            }
 #pragma unroll
             for (int j = 0; j < 2; j++) {
                 Acc s;
 #pragma unroll
                 for (int d = 0; d < kD; d++) s.add(xv[j][d], ev[j][d]);
+                if (ks.add) s.add(av[j], P.pmod);
                 const U128 v = s.get();
                 L[rl + 17 * (k0 + j)] = reduce128(v.hi, v.lo, br);
             }
@@ -612,11 +616,17 @@ __global__ __launch_bounds__(kTileThreads) void k_ntt_inv_b(uint64_t* data, JobS
 
 // The first inverse pass over a job list of ModDown limbs (off = pc E + t of an accumulator [n_polys][E][N]) whose
 // input is the evk inner product of a key switch of ciphertext pc / 2, poly pc % 2, formed here from the extension
-// [B][kD][E][N] and the key [dnum][2][T][N] (in place of a separate inner-product launch and its stores).
+// [B][kD][E][N] and the key [dnum][2][T][N] (in place of a separate inner-product launch and its stores).  With add (limb
+// t_add of the polys at add, add_pstride apart), limb t_add is the inner product + P add: a relinearization's addend joins
+// the dropped limb before its transform -- (x_{l-1} - conv) P^-1 + add and (x_{l-1} + P add - conv) P^-1 are the same
+// residue -- where its own transform had been two more launches (of 2 limbs a ciphertext: 15 us for one product).
 struct KsJobArgs {
     const uint64_t* ext;
     const uint64_t* evk;
     uint32_t E, T;
+    const uint64_t* add;
+    uint64_t add_pstride;
+    uint32_t t_add;
 };
 
 template <int kD, bool kCm>
@@ -628,7 +638,8 @@ __global__ __launch_bounds__(kTileThreads) void k_ntt_inv_b_ks(uint64_t* data, J
     const uint32_t pc = off / ka.E, t = off - pc * ka.E, c = pc >> 1, p = pc & 1;
     const PrimeInfo& P = primes[prime];
     const uint64_t* xin = ka.ext + ((size_t)c * kD * ka.E + t) * kN;
-    const KsIn ks{ka.evk + ((size_t)p * ka.T + prime) * kN, (size_t)ka.E * kN, 2 * (size_t)ka.T * kN};
+    const KsIn ks{ka.evk + ((size_t)p * ka.T + prime) * kN, (size_t)ka.E * kN, 2 * (size_t)ka.T * kN,
+                  ka.add && t == ka.t_add ? ka.add + pc * ka.add_pstride : nullptr};
     uint64_t* a = data + (size_t)off * kN;
     const TwPair* tw = tw_all + (size_t)prime * kN;
     const JobIn none{nullptr, nullptr};
@@ -1349,11 +1360,12 @@ hipError_t launch_ntt_fwd_ksl(const Context& ctx, uint64_t* y, const uint64_t* c
 
 // Inverse NTT of a job list over an accumulator [n_polys][E][N] (off = pc E + t) whose input, limb t of poly pc, is
 // the evk inner product sum_d ext[pc / 2][d][t] evk[d][pc % 2][prime] (the inner product a key switch would store
-// there first).  Digit counts 1..4 (others: hipErrorInvalidValue, the caller stores the inner product first).
+// there first); with add, limb t_add has P times add's added (see KsJobArgs).  Digit counts 1..4 (others: hipErrorInvalidValue, the caller stores the inner product first).
 hipError_t launch_ntt_inv_ks(const Context& ctx, uint64_t* acc, const JobSpec& js, uint32_t n_jobs,
-                             const uint64_t* ext, const uint64_t* evk, uint32_t D, uint32_t E, hipStream_t st) {
-    if (!js.jobs || D < 1 || D > 4 || n_jobs == 0) return hipErrorInvalidValue;
-    const KsJobArgs ka{ext, evk, E, ctx.L + ctx.K};
+                             const uint64_t* ext, const uint64_t* evk, uint32_t D, uint32_t E, hipStream_t st,
+                             const uint64_t* add, uint64_t add_pstride, uint32_t t_add) {
+    if (!js.jobs || D < 1 || D > 4 || n_jobs == 0 || (add && t_add >= ctx.L)) return hipErrorInvalidValue;
+    const KsJobArgs ka{ext, evk, E, ctx.L + ctx.K, add, add_pstride, t_add};
     // algorithmic bytes: per job D extension limbs read, the limb written, read back by the second pass and written
     // again; the key shared by the batch once: D limbs for each distinct (poly half, prime) of the jobs; the tables
     const double key_limbs = std::min<double>(n_jobs, 2.0 * js.n_primes) * D;

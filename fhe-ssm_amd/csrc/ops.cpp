@@ -51,7 +51,8 @@ hipError_t launch_ntt_inv_ksl(const Context& ctx, uint64_t* acc, const JobSpec& 
                               const uint64_t* const* ext, const uint64_t* const* evk, uint32_t n, uint32_t D,
                               uint32_t E, hipStream_t st);
 hipError_t launch_ntt_inv_ks(const Context& ctx, uint64_t* acc, const JobSpec& js, uint32_t n_jobs,
-                             const uint64_t* ext, const uint64_t* evk, uint32_t D, uint32_t E, hipStream_t st);
+                             const uint64_t* ext, const uint64_t* evk, uint32_t D, uint32_t E, hipStream_t st,
+                             const uint64_t* add = nullptr, uint64_t add_pstride = 0, uint32_t t_add = 0);
 hipError_t launch_ntt_fwd_sub(const Context& ctx, uint64_t* y, const uint64_t* x, uint64_t x_pstride,
                               const uint64_t* add, uint64_t add_pstride, uint32_t add_div, uint32_t add_group,
                               uint64_t* out, uint64_t out_pstride, uint32_t n_polys, uint32_t l, const TwPair* s,
@@ -767,13 +768,15 @@ void moddown_rescale(Context& ctx, uint64_t* x, uint32_t n_polys, uint32_t l, co
     const bool mf = mf_moddown(ctx, l);
     const MfRef r = mf ? mf_plan(ctx, kMfDownRescale, l, st) : MfRef{nullptr, nullptr};
     if (mf) js.scale = r.scale();
-    if (x_from_ext)  // those limbs of x are the evk inner product, formed by the transform's first pass
-        HIPX(launch_ntt_inv_ks(ctx, x, js, n_polys * (K + 1), ext, evk, num_digits(ctx, l), E, st));
+    if (x_from_ext)  // those limbs of x are the evk inner product (and P times the addend on limb l-1), formed by the
+                     // transform's first pass
+        HIPX(launch_ntt_inv_ks(ctx, x, js, n_polys * (K + 1), ext, evk, num_digits(ctx, l), E, st,
+                               add ? add + (size_t)(l - 1) * W : nullptr, (uint64_t)l * W, l - 1));
     else
         HIPX(launch_ntt(ctx, x, js, n_polys * (K + 1), true, ctx.ntt_mode, st));
-    // limb l-1 of the addend to coefficients (a copy: the addend is the caller's)
+    // otherwise limb l-1 of the addend to coefficients (a copy: the addend is the caller's)
     uint64_t* addc = nullptr;
-    if (add) {
+    if (add && !x_from_ext) {
         addc = (uint64_t*)ws_get(ctx, WS_LAST, (size_t)n_polys * W * 8);
         JobSpec ja = regular_jobs(n_polys, {l - 1});
         ja.src = add + (size_t)(l - 1) * W;
