@@ -86,7 +86,8 @@ hipError_t launch_automorph_list(const Context& ctx, const uint64_t* in, uint64_
                                  const uint32_t* g, hipStream_t st);
 hipError_t launch_bsgs_mac(const Context& ctx, const uint64_t* const* baby, const uint64_t* diag, uint64_t* out,
                            uint32_t nb, uint32_t n_diag, uint32_t ng, uint32_t l, uint32_t log_rep, hipStream_t st,
-                           uint32_t l_q = 0, uint32_t n_inst = 1, uint64_t inst_stride = 0, uint64_t out_stride = 0);
+                           uint32_t l_q = 0, uint32_t n_inst = 1, uint64_t inst_stride = 0, uint64_t out_stride = 0,
+                           uint32_t ngp = 1, int32_t g0 = -1, uint64_t* id_out = nullptr, uint64_t id_stride = 0);
 hipError_t launch_bsgs_dh_mac(const Context& ctx, const uint64_t* ext, uint64_t ext_stride, const uint64_t* src,
                               uint64_t src_stride, const uint64_t* const* keys, const uint32_t* g, uint32_t n_inst,
                               uint32_t n_in, uint32_t nb, const uint64_t* diag, uint32_t n_diag, uint32_t n_out,
@@ -1391,21 +1392,6 @@ void bsgs_multi_batch(Context& ctx, const uint64_t* const* in, uint32_t n_inst, 
         tmp = (uint64_t*)ws_get(ctx, WS_SUM, (size_t)n_x * nr * ctw * 8);
         rotate_hoisted_multi(ctx, X, n_x, l, rs.data(), nr, rk.data(), tmp, st);
     }
-    // babies [i nb + b] of instance s, read where they are (no packing copies)
-    std::vector<const uint64_t*> bp(nbt);
-    for (uint32_t s = 0; s < n_inst; s++) {
-        for (uint32_t i = 0; i < n_in; i++)
-            for (uint32_t b = 0; b < nb; b++) {
-                const size_t x = (size_t)s * n_in + i;
-                bp[i * nb + b] = ridx[b] < 0 ? X + x * ctw : tmp + (x * nr + (uint32_t)ridx[b]) * ctw;
-            }
-        HIPX(launch_bsgs_mac(ctx, bp.data(), diags, v + (size_t)s * n_out * ng * ctw, nbt, nbt * n_out * ng,
-                             n_out * ng, l, log_rep, st));
-    }
-    // the giant rotations share one ModDown per output: the rotating giant sums of every instance and output, packed
-    // contiguously, have their c1 extended (in chunks of outputs whose extensions fit a bounded buffer), and each
-    // output's sum_g Auto_g(<ext_g, evk_g> + (P c0_g, 0)) + P v_{g0} is formed in Q_l P by one kernel, placed at the
-    // output's slot; one ModDown (with the rescale) brings all outputs down
     const uint32_t n_o = n_inst * n_out;
     std::vector<const uint64_t*> gk;
     std::vector<uint32_t> gidx;
@@ -1420,13 +1406,31 @@ void bsgs_multi_batch(Context& ctx, const uint64_t* const* in, uint32_t n_inst, 
         gidx.push_back(rotation_index(gsteps[g]));
     }
     const uint32_t ngr = (uint32_t)gk.size();
+    // the rotating giant sums of every instance and output are written side by side (their c1 is extended as one strided
+    // batch), the identity giant's after them
+    uint64_t* v_id = v + (size_t)n_o * ngr * ctw;
+    // babies [i nb + b] of instance s, read where they are (no packing copies)
+    std::vector<const uint64_t*> bp(nbt);
+    for (uint32_t s = 0; s < n_inst; s++) {
+        for (uint32_t i = 0; i < n_in; i++)
+            for (uint32_t b = 0; b < nb; b++) {
+                const size_t x = (size_t)s * n_in + i;
+                bp[i * nb + b] = ridx[b] < 0 ? X + x * ctw : tmp + (x * nr + (uint32_t)ridx[b]) * ctw;
+            }
+        HIPX(launch_bsgs_mac(ctx, bp.data(), diags, v + (size_t)s * n_out * ngr * ctw, nbt, nbt * n_out * ng,
+                             n_out * ng, l, log_rep, st, 0, 1, 0, 0, ng, g0, v_id + (size_t)s * n_out * ctw, ctw));
+    }
+    // the giant rotations share one ModDown per output: the rotating giant sums of every instance and output, side by
+    // side, have their c1 extended (in chunks of outputs whose extensions fit a bounded buffer), and each
+    // output's sum_g Auto_g(<ext_g, evk_g> + (P c0_g, 0)) + P v_{g0} is formed in Q_l P by one kernel, placed at the
+    // output's slot; one ModDown (with the rescale) brings all outputs down
     const auto slot_of = [&](uint32_t c) {  // output c = s n_out + o -> its place in out
         return by_output ? (size_t)(c % n_out) * n_inst + c / n_out : (size_t)c;
     };
     if (ngr == 0) {  // the identity giant only: its sums are the outputs
         uint64_t* dst = do_rescale ? (uint64_t*)ws_get(ctx, WS_LIN, (size_t)n_o * ctw * 8) : out;
         for (uint32_t c = 0; c < n_o; c++) {
-            const uint64_t* term = v + ((size_t)c * ng + (uint32_t)g0) * ctw;
+            const uint64_t* term = v_id + (size_t)c * ctw;
             HIPX(launch_sum_list(ctx, &term, 1, dst + slot_of(c) * ctw, 2, l, st));
         }
         if (do_rescale) rescale(ctx, dst, 2 * n_o, l, out, st);
@@ -1434,30 +1438,21 @@ void bsgs_multi_batch(Context& ctx, const uint64_t* const* in, uint32_t n_inst, 
     }
     const uint32_t E = l + ctx.K, D = num_digits(ctx, l);
     const size_t exw = (size_t)D * E * W, cte = (size_t)2 * E * W;
-    uint64_t* packed = (uint64_t*)ws_get(ctx, WS_SUM, (size_t)n_o * ngr * ctw * 8);
-    {
-        std::vector<const uint64_t*> src;
-        src.reserve((size_t)n_o * ngr);
-        for (uint32_t c = 0; c < n_o; c++)
-            for (uint32_t g = 0; g < ng; g++)
-                if ((int32_t)g != g0) src.push_back(v + ((size_t)c * ng + g) * ctw);
-        HIPX(launch_gather(ctx, src.data(), (uint32_t)src.size(), ctw, packed, st));
-    }
     uint64_t* T = (uint64_t*)ws_get(ctx, WS_GROT, (size_t)n_o * cte * 8);
     const uint32_t chunk = std::max<uint32_t>(1, 32 / ngr);
     uint64_t* ext = (uint64_t*)ws_get(ctx, WS_EXT, (size_t)std::min(chunk, n_o) * ngr * exw * 8);
     const TwPair* pm = pmod_tab(ctx).data();
     for (uint32_t o0 = 0; o0 < n_o; o0 += chunk) {
         const uint32_t m = std::min(chunk, n_o - o0);
-        const uint64_t* src = packed + (size_t)o0 * ngr * ctw;
+        const uint64_t* src = v + (size_t)o0 * ngr * ctw;
         modup(ctx, src + (size_t)l * W, ext, m * ngr, l, st, ctw);
-        const uint64_t* id = g0 >= 0 ? v + ((size_t)o0 * ng + (uint32_t)g0) * ctw : nullptr;
+        const uint64_t* id = g0 >= 0 ? v_id + (size_t)o0 * ctw : nullptr;
         if (by_output)
             HIPX(launch_qp_rot_sum(ctx, ext, exw, src, ctw, gk.data(), gidx.data(), m, ngr, 1, ngr, l, T, st, n_out, o0,
-                                   (uint64_t)n_inst * cte, false, pm, id, (uint64_t)ng * ctw));
+                                   (uint64_t)n_inst * cte, false, pm, id, ctw));
         else
             HIPX(launch_qp_rot_sum(ctx, ext, exw, src, ctw, gk.data(), gidx.data(), m, ngr, 1, ngr, l,
-                                   T + (size_t)o0 * cte, st, 1, 0, 0, false, pm, id, (uint64_t)ng * ctw));
+                                   T + (size_t)o0 * cte, st, 1, 0, 0, false, pm, id, ctw));
     }
     if (do_rescale)
         moddown_rescale(ctx, T, 2 * n_o, l, nullptr, out, st);

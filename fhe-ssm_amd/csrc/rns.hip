@@ -691,26 +691,27 @@ struct GiantMap {
     int32_t g0;
     uint64_t* id_out;
     uint64_t id_stride;
+
+    // where giant sum g of [2][..] words is stored (stride words apart in out)
+    __device__ __forceinline__ uint64_t* place(uint64_t* out, uint32_t g, size_t stride) const {
+        if (g0 < 0) return out + g * stride;
+        const uint32_t oi = g / ngp, gi = g - oi * ngp;
+        if (gi == (uint32_t)g0) return id_out + (size_t)oi * id_stride;
+        return out + ((size_t)oi * (ngp - 1) + gi - (gi > (uint32_t)g0 ? 1 : 0)) * stride;
+    }
 };
 
 __device__ __forceinline__ void mac_giants(const uint64_t* sb, const uint64_t* __restrict__ diag,
                                            uint64_t* __restrict__ out, uint32_t nb, uint32_t nb_total, uint32_t j0,
                                            uint32_t ng, uint32_t n_diag, size_t P, size_t Pd, size_t dk, size_t off,
                                            uint32_t acc, const Barrett& br, uint32_t kk, uint32_t row,
-                                           const GiantMap& gm = GiantMap{1, -1, nullptr, 0}) {
+                                           const GiantMap& gm) {
     auto count = [&](uint32_t g) {
         const int64_t rem = (int64_t)n_diag - (int64_t)g * nb_total - j0;
         return rem <= 0 ? 0u : (uint32_t)min<int64_t>(rem, nb);
     };
     auto store = [&](uint32_t g, Acc& a0, Acc& a1) {
-        uint64_t* o = out + (size_t)g * 2 * P + off;
-        if (gm.g0 >= 0) {
-            const uint32_t oi = g / gm.ngp, gi = g - oi * gm.ngp;
-            if (gi == (uint32_t)gm.g0)
-                o = gm.id_out + (size_t)oi * gm.id_stride + off;
-            else
-                o = out + ((size_t)oi * (gm.ngp - 1) + gi - (gi > (uint32_t)gm.g0 ? 1 : 0)) * 2 * P + off;
-        }
+        uint64_t* o = gm.place(out, g, 2 * P) + off;
         uint64_t r0 = reduce_u128(a0.get(), br), r1 = reduce_u128(a1.get(), br);
         if (acc) {
             r0 = add_mod(r0, o[0], br.q);
@@ -780,6 +781,7 @@ __device__ __forceinline__ void mac_giants(const uint64_t* sb, const uint64_t* _
 // n_inst instances share the diagonals: instance s takes its babies at baby.p[j] + s inst_stride and writes
 // out + s out_stride; the instances of one (coefficient tile, limb) run on one XCD (list_tile), so each diagonal
 // word is fetched from HBM once for all of them.
+// gm places the giant sums.
 __global__ __launch_bounds__(kMacCoef* kMacRows) void k_bsgs_mac(ListPtrs baby,
                                                                   const uint64_t* __restrict__ diag,
                                                                   uint64_t* __restrict__ out, uint32_t nb,
@@ -787,7 +789,7 @@ __global__ __launch_bounds__(kMacCoef* kMacRows) void k_bsgs_mac(ListPtrs baby,
                                                                   uint32_t n_diag, uint32_t l, uint32_t log_rep,
                                                                   uint32_t acc, uint32_t l_q, uint32_t Lp,
                                                                   uint32_t n_inst, uint64_t inst_stride,
-                                                                  uint64_t out_stride,
+                                                                  uint64_t out_stride, GiantMap gm,
                                                                   const PrimeInfo* __restrict__ primes) {
     extern __shared__ uint64_t sb[];
     const ListTile lt = list_tile(n_inst, kN / kMacCoef);
@@ -806,7 +808,7 @@ __global__ __launch_bounds__(kMacCoef* kMacRows) void k_bsgs_mac(ListPtrs baby,
     }
     __syncthreads();
     mac_giants(sb, diag, out, nb, nb_total, j0, ng, n_diag, P, (size_t)l * (kN >> log_rep),
-               (size_t)i * (kN >> log_rep) + (k >> log_rep), off, acc, br, kk, row);
+               (size_t)i * (kN >> log_rep) + (k >> log_rep), off, acc, br, kk, row, gm);
 }
 
 // Double-hoisted BSGS MAC: the babies are formed in LDS from the inputs' ModUp extensions and never stored.  Over
@@ -1318,7 +1320,10 @@ hipError_t launch_automorph_list(const Context& ctx, const uint64_t* in, uint64_
 // l limbs per poly; with l_q < l the limbs from l_q on are the P limbs (an extended-basis MAC)
 hipError_t launch_bsgs_mac(const Context& ctx, const uint64_t* const* baby, const uint64_t* diag, uint64_t* out,
                            uint32_t nb, uint32_t n_diag, uint32_t ng, uint32_t l, uint32_t log_rep, hipStream_t st,
-                           uint32_t l_q, uint32_t n_inst, uint64_t inst_stride, uint64_t out_stride) {
+                           uint32_t l_q, uint32_t n_inst, uint64_t inst_stride, uint64_t out_stride, uint32_t ngp,
+                           int32_t g0, uint64_t* id_out, uint64_t id_stride) {
+    const GiantMap gm{ngp, g0, id_out, id_stride};
+    if (ngp == 0 || (g0 >= 0 && (!id_out || g0 >= (int32_t)ngp))) return hipErrorInvalidValue;
     if (l_q == 0 || l_q > l) l_q = l;
     if (nb == 0 || log_rep > 6 || n_diag > nb * ng || n_inst == 0 || n_inst > 4096) return hipErrorInvalidValue;
     const double bytes =
@@ -1330,7 +1335,7 @@ hipError_t launch_bsgs_mac(const Context& ctx, const uint64_t* const* baby, cons
         for (uint32_t j = 0; j < nbc; j++) bp.p[j] = baby[j0 + j];
         hipLaunchKernelGGL(k_bsgs_mac, dim3(n_inst * (kN / kMacCoef) * l), dim3(kMacCoef * kMacRows),
                            (size_t)nbc * 2 * kMacCoef * 8, st, bp, diag, out, nbc, nb, j0, ng, n_diag, l, log_rep,
-                           j0 ? 1u : 0u, l_q, ctx.L, n_inst, inst_stride, out_stride, ctx.d_primes);
+                           j0 ? 1u : 0u, l_q, ctx.L, n_inst, inst_stride, out_stride, gm, ctx.d_primes);
     }
     prof_end(ctx, pi, st);
     return hipGetLastError();
