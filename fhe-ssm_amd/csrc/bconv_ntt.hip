@@ -85,7 +85,7 @@ __device__ __forceinline__ void mf_words(uint64_t* x, const uint64_t* base, cons
     for (int s = 0; s < KS; s++)
 #pragma unroll
         for (int t = 0; t < 2; t++) a[s][t] = A[(s * 2 + t) * 64];
-    constexpr int kB = KS == 2 ? 4 : kExtra ? 8 : 16;  // rows whose words are requested together (as registers allow)
+    constexpr int kB = KS == 2 || kExtra ? 8 : 16;  // rows whose words are requested together (as registers allow)
 #pragma unroll
     for (int k0 = 0; k0 < 16; k0 += kB) {
         uint64_t y[kB][KS][2], e[kB];
@@ -219,9 +219,11 @@ __device__ __forceinline__ void bc_column(const uint64_t* __restrict__ in, const
 
 // grid: 64 quads of columns x (groups of 4 outputs of every digit) x batch, one dimension.  Workgroups go to the 8 XCDs
 // round-robin; id = xcd + 8 s, and XCD xcd takes the columns [32 xcd, 32 xcd + 32), s running over their 8 quads fastest,
-// then the groups (which read the same source words, kept by that XCD's L2), then the batch.
+// then the groups (which read the same source words, kept by that XCD's L2), then the batch.  Two steps of source limbs
+// take 136 registers: three waves a SIMD without spills and 8 rows' words in flight (11 conversions of 9 -> 25 limbs
+// 436 us) against four with 3 spilled and 4 rows' (464).
 template <int KS, bool kTail, bool kExtra>
-__global__ __launch_bounds__(64 * kBcWaves) __attribute__((amdgpu_waves_per_eu(4))) void k_bconv_ntt_a(
+__global__ __launch_bounds__(64 * kBcWaves) __attribute__((amdgpu_waves_per_eu(KS == 2 ? 3 : 4))) void k_bconv_ntt_a(
     const uint64_t* __restrict__ in, const uint64_t* __restrict__ extra, uint64_t* __restrict__ out, MfArgs ma,
     const TwPair* __restrict__ twa) {
     __shared__ BcShared shared[kBcWaves];
