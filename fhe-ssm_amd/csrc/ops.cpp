@@ -394,16 +394,42 @@ static void check_level(const Context& ctx, uint32_t l) {
 }
 
 // ------------------------------------------------------------------ matrix-core conversions
-// Taken under the two-pass NTT for every chain whose primes have at least 35 bits (the reduction's quotient unit) and
-// conversions within the tables' limits; otherwise k_bconv and a whole forward NTT.
+// Possible under the two-pass NTT for every chain whose primes have at least 35 bits (the reduction's quotient unit) and
+// conversions within the tables' limits; otherwise, and where it is the slower form, k_bconv and a whole forward NTT.
+// It forms its outputs in groups of four and every output's butterflies at once, so a conversion of one or two outputs
+// does up to four times the work; and where all source limbs of a coefficient are needed at once (exact rounding, the
+// rescale) it adds a launch that reads them again (k_moddown_head), which few outputs cannot pay for.  The lines below
+// are where the two forms cross, measured on whole calls over K = 1..16, 1..24 limbs and 1..128 polys; a percentage is
+// the matrix-core form's time over the other's.
 enum MfKind : uint32_t { kMfModUp = 0, kMfDown = 1, kMfDownRescale = 2 };
 
-static bool mf_modup(const Context& ctx, uint32_t l) {
-    return ctx.ntt_mode == NttMode::TwoPass && ctx.mf_primes && ctx.alpha <= (uint32_t)kMfMaxIn &&
-           l + ctx.K <= kMfMaxOut;
+// ModUp of B polys: slower only for a few outputs of many polys with one or two special primes (K = 1, 1 limb, 32 polys
+// +23%; K = 2, 1 limb +8%, 2 limbs +5%; but K = 3, 1 limb -2%, and K = 8, 1 to 24 limbs -14% to -26%).
+static bool mf_modup(const Context& ctx, uint32_t l, uint32_t B) {
+    if (ctx.ntt_mode != NttMode::TwoPass || !ctx.mf_primes || ctx.alpha > (uint32_t)kMfMaxIn || l + ctx.K > kMfMaxOut)
+        return false;
+    const uint32_t D = (l + ctx.alpha - 1) / ctx.alpha, n_out = D * (l + ctx.K) - l;  // outputs of all digits
+    return ctx.K >= 3 || n_out >= 8 || B < 16;
 }
-static bool mf_moddown(const Context& ctx, uint32_t l) {
-    return ctx.ntt_mode == NttMode::TwoPass && ctx.mf_primes && ctx.K <= (uint32_t)kMfMaxIn && l <= kMfMaxOut;
+
+// ModDown to l limbs of n_polys polys.
+static bool mf_moddown(const Context& ctx, uint32_t kind, uint32_t l, uint32_t n_polys, bool list) {
+    if (ctx.ntt_mode != NttMode::TwoPass || !ctx.mf_primes || ctx.K > (uint32_t)kMfMaxIn || l > kMfMaxOut) return false;
+    // with the rescale: K = 8, product of 32 pairs to 2 limbs +8%, 4 limbs +4%, 8 limbs +-1%, 16 limbs -2%, 24 -3%; of one
+    // pair 2 limbs +-1%, 5 limbs -3%, 24 limbs -10%
+    if (kind == kMfDownRescale) return l >= (n_polys >= 16 ? 8u : 3u);
+    if (ctx.moddown_exact) {
+        // of a key-switch list: K = 8, 32 items 3 limbs +6%, 6 limbs +2%, 8 limbs -1%, 24 limbs -4%; one item 2 limbs +1%,
+        // 4 limbs -2%
+        if (list) return l >= (n_polys > 16 ? 8u : 4u);
+        // alone: K = 8, 2 polys 8 limbs +7%, 11 limbs +5%, 16 limbs -7%; 8 polys 4 limbs +-0, 8 limbs -3%; 64 polys 5 limbs
+        // +8%, 8 limbs -1%; K = 2, 8 polys 8 limbs +6%, 11 limbs +1%, 24 polys 8 limbs -6%
+        return l >= 12 || (l >= 8 && n_polys * ctx.K >= 48);
+    }
+    // 1 limb, 64 polys: K = 1 +23%, K = 7 +7%, K = 8 -2%, K = 16 +2%; 8 polys or fewer of any K -6% to +1%.  2 limbs: K = 2,
+    // 128 polys alone +4%, in a list -1%, 16 polys -4%; K = 3 -1%, K = 8 -3%.  3 limbs: -4% to -10%
+    if (l == 1) return n_polys <= 8 || ctx.K % 8 == 0;
+    return l >= 3 || list || ctx.K >= 3 || n_polys <= 16;
 }
 
 // prod of the primes idx but idx[skip], mod q
@@ -587,8 +613,8 @@ static void mf_convert(Context& ctx, const MfRef& r, const uint64_t* in, uint64_
 
 // ------------------------------------------------------------------ ModUp
 // the factors the inverse NTT of a ModUp source folds into its last stage (null: plain coefficients)
-static const InvScale* modup_scale(Context& ctx, uint32_t l, hipStream_t st) {
-    return mf_modup(ctx, l) ? mf_plan(ctx, kMfModUp, l, st).scale() : nullptr;
+static const InvScale* modup_scale(Context& ctx, uint32_t l, uint32_t B, hipStream_t st) {
+    return mf_modup(ctx, l, B) ? mf_plan(ctx, kMfModUp, l, st).scale() : nullptr;
 }
 
 // x2c: [B][l][N] inverse NTT (with modup_scale's factors) of the polynomial to extend;
@@ -596,7 +622,7 @@ static const InvScale* modup_scale(Context& ctx, uint32_t l, hipStream_t st) {
 // evaluation form, or their consumer forms them).
 void modup_from_coef(Context& ctx, const uint64_t* x2c, uint64_t* ext, uint32_t B, uint32_t l, hipStream_t st) {
     const uint32_t D = num_digits(ctx, l), E = l + ctx.K, al = ctx.alpha;
-    const bool mf = mf_modup(ctx, l);
+    const bool mf = mf_modup(ctx, l, B);
     std::vector<Job> jobs;
     for (uint32_t d = 0; d < D; d++) {
         const uint32_t lo = d * al, hi = std::min(lo + al, l);
@@ -649,7 +675,7 @@ void modup(Context& ctx, const uint64_t* x, uint64_t* ext, uint32_t B, uint32_t 
     js.copy_pstride = (uint64_t)D * E * W;
     js.copy_alpha = al;
     js.copy_E = E;
-    js.scale = modup_scale(ctx, l, st);
+    js.scale = modup_scale(ctx, l, B, st);
     HIPX(launch_ntt(ctx, xc, js, B * l, true, ctx.ntt_mode, st));
     modup_from_coef(ctx, xc, ext, B, l, st);
 }
@@ -704,7 +730,7 @@ void moddown_inplace(Context& ctx, uint64_t* x, uint32_t n_polys, uint32_t l, co
                              std::move(jobs));
     uint64_t* conv = (uint64_t*)ws_get(ctx, WS_CONV, (size_t)n_polys * l * W * 8);
     const uint64_t aps = add_pstride < 0 ? (uint64_t)add_div * l * W : (uint64_t)add_pstride;
-    if (mf_moddown(ctx, l)) {
+    if (mf_moddown(ctx, kMfDown, l, n_polys, false)) {
         const MfRef r = mf_plan(ctx, kMfDown, l, st);
         js.scale = r.scale();
         HIPX(launch_ntt(ctx, x, js, n_polys * K, true, ctx.ntt_mode, st));
@@ -766,7 +792,7 @@ void moddown_rescale(Context& ctx, uint64_t* x, uint32_t n_polys, uint32_t l, co
         for (uint32_t k = 0; k < K; k++) jobs.push_back(Job{pc * E + l + k, ctx.L + k});
     }
     JobSpec js = cached_jobs(ctx, "mdrP:" + std::to_string(n_polys) + ":" + std::to_string(l), std::move(jobs));
-    const bool mf = mf_moddown(ctx, l);
+    const bool mf = mf_moddown(ctx, kMfDownRescale, l, n_polys, false);
     const MfRef r = mf ? mf_plan(ctx, kMfDownRescale, l, st) : MfRef{nullptr, nullptr};
     if (mf) js.scale = r.scale();
     if (x_from_ext)  // those limbs of x are the evk inner product (and P times the addend on limb l-1), formed by the
@@ -875,7 +901,7 @@ void ks_moddown_list(Context& ctx, const uint64_t* const* ext, const uint64_t* c
     for (uint32_t pc = 0; pc < 2 * n; pc++)
         for (uint32_t k = 0; k < K; k++) jobs.push_back(Job{pc * E + l + k, ctx.L + k});
     JobSpec js = cached_jobs(ctx, "mdP:" + std::to_string(2 * n) + ":" + std::to_string(l), std::move(jobs));
-    const bool mf = mf_moddown(ctx, l);
+    const bool mf = mf_moddown(ctx, kMfDown, l, 2 * n, true);
     const MfRef r = mf ? mf_plan(ctx, kMfDown, l, st) : MfRef{nullptr, nullptr};
     if (mf) js.scale = r.scale();
     if (fused) {
@@ -1030,7 +1056,7 @@ static void relin_tail(Context& ctx, uint64_t* d01, uint64_t* x2c, uint64_t* ext
     for (uint32_t i = 0; i < l; i++) pm[i] = i;
     if (!x2c_coef) {
         JobSpec js = regular_jobs(B, pm);
-        js.scale = modup_scale(ctx, l, st);
+        js.scale = modup_scale(ctx, l, B, st);
         HIPX(launch_ntt(ctx, x2c, js, B * l, true, ctx.ntt_mode, st));
     }
     modup_from_coef(ctx, x2c, ext, B, l, st);
@@ -1083,7 +1109,7 @@ void hmult(Context& ctx, const uint64_t* a, const uint64_t* b, uint32_t B, uint3
     js.copy_alpha = ctx.alpha;
     js.copy_E = E;
     js.copy_from = own ? l - 1 : 0;
-    js.scale = modup_scale(ctx, l, st);
+    js.scale = modup_scale(ctx, l, B, st);
     HIPX(launch_ntt(ctx, x2c, js, B * l, true, ctx.ntt_mode, st));
     if (from_inputs)
         relin_tail(ctx, d01, x2c, ext, B, l, evk, out, true, st, a, b, true, aff, own);
