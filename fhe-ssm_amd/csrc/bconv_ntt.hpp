@@ -4,7 +4,6 @@
 
 namespace fhe {
 
-constexpr int kMfMaxIn = 16;        // source limbs of a conversion
 constexpr uint32_t kMfMaxOut = 80;  // output limbs of a conversion
 constexpr uint32_t kMfMaxDigits = 8;
 // the quotient estimate of the reduction needs primes of at least 35 bits (its unit is 2^32)
@@ -35,13 +34,6 @@ struct MfArgs {
     MfDigit dig[kMfMaxDigits];
     uint32_t n_dig, n_grp;  // conversions, their groups in all
     uint64_t in_bstride, out_bstride, extra_bstride;
-};
-
-struct MfHeadArgs {
-    uint32_t n_in, exact, rescale, last;
-    uint64_t c[kMfMaxIn + 1];    // column of the dropped limb, then -P mod q_{l-1}
-    uint64_t fix[kMfMaxIn][2];   // floor(2^128 / p_i), low and high word
-    TwPair pinv;                 // P^-1 mod q_{l-1}
 };
 
 hipError_t launch_bconv_ntt_a(const Context& ctx, uint32_t ks, const uint64_t* in, const uint64_t* extra, uint64_t* out,

@@ -102,9 +102,20 @@ struct MfConv {
     uint64_t in_off, out_off;          // words from a batch item's base
 };
 
+constexpr int kMfMaxIn = 16;  // source limbs of a conversion
+
+// k_moddown_head's constants (exact is set by the call)
+struct MfHeadArgs {
+    uint32_t n_in, exact, rescale, last;
+    uint64_t c[kMfMaxIn + 1];   // with the rescale: column of the dropped limb, then -P mod q_{l-1}
+    uint64_t fix[kMfMaxIn][2];  // floor(2^128 / p_i), low and high word
+    TwPair pinv;                // P^-1 mod q_{l-1}
+};
+
 struct MfPlan {
     uint32_t ks = 1, n_grp = 0;
     std::vector<MfConv> conv;
+    MfHeadArgs head{};  // of a ModDown
     std::vector<uint64_t> host;
     size_t words = 0;
     uint64_t* dev = nullptr;  // null: built for allocation-free calls only (their arena holds the device copy)

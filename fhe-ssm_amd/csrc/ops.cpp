@@ -534,6 +534,21 @@ static MfPlan mf_build(const Context& ctx, uint32_t kind, uint32_t l) {
             mf_put(p.host, (size_t)(l - 1) * (sizeof(InvScale) / 8), &sc, sizeof(sc));
         }
         mf_add(ctx, p, in_idx, out_idx, out_idx, (uint64_t)l * W, 0, col);
+        MfHeadArgs& ha = p.head;
+        ha.n_in = ctx.K;
+        ha.rescale = rescale ? 1 : 0;
+        ha.last = l - 1;
+        for (uint32_t k = 0; k < ctx.K; k++) {
+            const unsigned __int128 c = (~(unsigned __int128)0) / ctx.moduli[ctx.L + k];  // floor(2^128 / p_k)
+            ha.fix[k][0] = (uint64_t)c;
+            ha.fix[k][1] = (uint64_t)(c >> 64);
+        }
+        if (rescale) {
+            const uint64_t ql = ctx.moduli[l - 1], P = prod_mod(ctx, in_idx, in_idx.size(), ql), v = invmod_h(P, ql);
+            for (uint32_t k = 0; k < ctx.K; k++) ha.c[k] = prod_mod(ctx, in_idx, k, ql);
+            ha.c[kMfMaxIn] = ql - P;
+            ha.pinv = TwPair{v, shoup_companion(v, ql)};
+        }
     }
     p.words = (p.host.size() + 1) & ~(size_t)1;  // the operands are read 16 bytes at a time
     for (auto& c : p.conv) {
@@ -687,28 +702,13 @@ void ks_inner(Context& ctx, const uint64_t* ext, const uint64_t* evk, uint64_t* 
     HIPX(launch_ks_inner(ctx, ext, evk, acc, B, l, st));
 }
 
-// the limb added in a ModDown conversion (k_moddown_head) from the P limbs' digit words y: with the rescale, limb l-1 of
-// the polys (coefficients, at xlast) and of the addend (addc, or null) enter it
-static void moddown_head(Context& ctx, const uint64_t* y, uint64_t y_bstride, uint64_t* e, uint64_t e_bstride, uint32_t l,
-                         bool rescale, const uint64_t* xlast, uint64_t x_bstride, const uint64_t* addc, uint32_t n_polys,
-                         hipStream_t st) {
-    MfHeadArgs ha{};
-    ha.n_in = ctx.K;
+// the limb added in a ModDown conversion (k_moddown_head) from the P limbs' digit words y: with the rescale (by the plan),
+// limb l-1 of the polys (coefficients, at xlast) and of the addend (addc, or null) enter it
+static void moddown_head(Context& ctx, const MfPlan& p, const uint64_t* y, uint64_t y_bstride, uint64_t* e,
+                         uint64_t e_bstride, const uint64_t* xlast, uint64_t x_bstride, const uint64_t* addc,
+                         uint32_t n_polys, hipStream_t st) {
+    MfHeadArgs ha = p.head;
     ha.exact = ctx.moddown_exact ? 1 : 0;
-    ha.rescale = rescale ? 1 : 0;
-    ha.last = l - 1;
-    std::vector<uint32_t> in_idx;
-    for (uint32_t k = 0; k < ctx.K; k++) in_idx.push_back(ctx.L + k);
-    const uint64_t ql = ctx.moduli[l - 1];
-    for (uint32_t k = 0; k < ctx.K; k++) {
-        const unsigned __int128 c = (~(unsigned __int128)0) / ctx.moduli[ctx.L + k];  // floor(2^128 / p_k)
-        ha.fix[k][0] = (uint64_t)c;
-        ha.fix[k][1] = (uint64_t)(c >> 64);
-        ha.c[k] = prod_mod(ctx, in_idx, k, ql);
-    }
-    const uint64_t P = prod_mod(ctx, in_idx, in_idx.size(), ql);
-    ha.c[kMfMaxIn] = P ? ql - P : 0;
-    ha.pinv = pinv_tab(ctx)[l - 1];
     HIPX(launch_moddown_head(ctx, y, y_bstride, e, e_bstride, xlast, x_bstride, addc, ha, n_polys, st));
 }
 
@@ -737,7 +737,7 @@ void moddown_inplace(Context& ctx, uint64_t* x, uint32_t n_polys, uint32_t l, co
         uint64_t* e = nullptr;
         if (ctx.moddown_exact) {
             e = (uint64_t*)ws_get(ctx, WS_LAST, (size_t)n_polys * W * 8);
-            moddown_head(ctx, x + (size_t)l * W, (uint64_t)xs * W, e, W, l, false, nullptr, 0, nullptr, n_polys, st);
+            moddown_head(ctx, *r.plan, x + (size_t)l * W, (uint64_t)xs * W, e, W, nullptr, 0, nullptr, n_polys, st);
         }
         mf_convert(ctx, r, x, (uint64_t)xs * W, e, W, conv, (uint64_t)l * W, n_polys, st);
         HIPX(launch_ntt_fwd_sub(ctx, conv, x, (uint64_t)xs * W, add, aps, add_div, add_group, out, (uint64_t)l * W,
@@ -811,28 +811,25 @@ void moddown_rescale(Context& ctx, uint64_t* x, uint32_t n_polys, uint32_t l, co
         if (mf) ja.scale = r.scale();
         HIPX(launch_ntt(ctx, addc, ja, n_polys, true, ctx.ntt_mode, st));
     }
-    const std::vector<TwPair>& ptab = pinv_tab(ctx);
-    const std::vector<TwPair>& qrow = qinv_row(ctx, l - 1);
-    std::vector<TwPair> pinv(ptab.begin(), ptab.begin() + l), qlinv(l);
-    std::vector<uint64_t> col(l);
-    for (uint32_t i = 0; i < l; i++) {
-        col[i] = i + 1 < l ? pinv[i].w : 1;  // columns 0..l-2 carry P^-1; the dropped limb's column stays plain
-        qlinv[i] = i + 1 < l ? qrow[i] : TwPair{0, 0};
-    }
-    std::vector<uint32_t> in_idx, in_off, out_idx;
-    for (uint32_t k = 0; k < K; k++) {
-        in_idx.push_back(ctx.L + k);
-        in_off.push_back(l + k);
-    }
-    for (uint32_t i = 0; i < l; i++) out_idx.push_back(i);
+    const std::vector<TwPair>&pinv = pinv_tab(ctx), &qlinv = qinv_row(ctx, l - 1);
     uint64_t* T = (uint64_t*)ws_get(ctx, WS_RTMP, (size_t)n_polys * (l - 1) * W * 8);
     const uint64_t xps = (uint64_t)E * W;
     if (mf) {
         // the limb to add takes the place of limb l-1 of x
         uint64_t* e = x + (size_t)(l - 1) * W;
-        moddown_head(ctx, x + (size_t)l * W, xps, e, xps, l, true, e, xps, addc, n_polys, st);
+        moddown_head(ctx, *r.plan, x + (size_t)l * W, xps, e, xps, e, xps, addc, n_polys, st);
         mf_convert(ctx, r, x, xps, e, xps, T, (uint64_t)(l - 1) * W, n_polys, st, "bconv_mdr");
     } else {
+        std::vector<uint32_t> in_idx, in_off, out_idx;
+        for (uint32_t k = 0; k < K; k++) {
+            in_idx.push_back(ctx.L + k);
+            in_off.push_back(l + k);
+        }
+        std::vector<uint64_t> col(l, 1);  // columns 0..l-2 carry P^-1; the dropped limb's column stays plain
+        for (uint32_t i = 0; i < l; i++) {
+            out_idx.push_back(i);
+            if (i + 1 < l) col[i] = pinv[i].w;
+        }
         const BConvPlan& plan = bconv_plan(ctx, in_idx, out_idx, ctx.moddown_exact, col);
         HIPX(launch_bconv_mdr(ctx, plan, x, xps, in_off.data(), T, n_polys, x + (size_t)(l - 1) * W, xps, addc,
                               pinv[l - 1], st));
@@ -912,24 +909,25 @@ void ks_moddown_list(Context& ctx, const uint64_t* const* ext, const uint64_t* c
         HIPX(launch_ks_inner_list(ctx, ext, evk, acc, n, l, st, l));
         HIPX(launch_ntt(ctx, acc, js, 2 * n * K, true, ctx.ntt_mode, st));
     }
-    std::vector<uint32_t> in_idx, in_off, out_idx;
-    for (uint32_t k = 0; k < K; k++) {
-        in_idx.push_back(ctx.L + k);
-        in_off.push_back(l + k);
-    }
-    const std::vector<TwPair> pinv(pinv_tab(ctx).begin(), pinv_tab(ctx).begin() + l);
-    std::vector<uint64_t> col(l);
-    for (uint32_t i = 0; i < l; i++) {
-        out_idx.push_back(i);
-        col[i] = pinv[i].w;
-    }
+    const std::vector<TwPair>& pinv = pinv_tab(ctx);
+    std::vector<uint32_t> out_idx(l);
+    for (uint32_t i = 0; i < l; i++) out_idx[i] = i;
     uint64_t* conv = (uint64_t*)ws_get(ctx, WS_CONV, (size_t)2 * n * l * W * 8);
     if (mf) {
         // the limb to add (exact form) in limb l-1 of the accumulator, whose Q limbs are never formed
         uint64_t* e = ctx.moddown_exact ? acc + (size_t)(l - 1) * W : nullptr;
-        if (e) moddown_head(ctx, acc + (size_t)l * W, (uint64_t)E * W, e, (uint64_t)E * W, l, false, nullptr, 0, nullptr, 2 * n, st);
+        if (e)
+            moddown_head(ctx, *r.plan, acc + (size_t)l * W, (uint64_t)E * W, e, (uint64_t)E * W, nullptr, 0, nullptr, 2 * n,
+                         st);
         mf_convert(ctx, r, acc, (uint64_t)E * W, e, (uint64_t)E * W, conv, (uint64_t)l * W, 2 * n, st);
     } else {
+        std::vector<uint32_t> in_idx, in_off;
+        for (uint32_t k = 0; k < K; k++) {
+            in_idx.push_back(ctx.L + k);
+            in_off.push_back(l + k);
+        }
+        std::vector<uint64_t> col(l);
+        for (uint32_t i = 0; i < l; i++) col[i] = pinv[i].w;
         const BConvPlan& plan = bconv_plan(ctx, in_idx, out_idx, ctx.moddown_exact, col);
         HIPX(launch_bconv(ctx, plan, acc, (uint64_t)E * W, in_off.data(), conv, (uint64_t)l * W, out_idx.data(), 2 * n,
                           st));

@@ -1429,7 +1429,7 @@ static MdrArgs mdr_args(uint32_t l, uint64_t x_pstride, uint64_t add_pstride, co
     ma.l = l;
     ma.x_pstride = x_pstride;
     ma.add_pstride = add_pstride;
-    for (uint32_t i = 0; i < l; i++) {
+    for (uint32_t i = 0; i + 1 < l; i++) {  // the limbs kept
         ma.pinv[i] = pinv[i];
         ma.qlinv[i] = qlinv[i];
     }
