@@ -328,14 +328,14 @@ hipError_t launch_bconv_ntt_a(const Context& ctx, uint32_t ks, const uint64_t* i
     if (ks < 1 || ks > 2 || ma.n_dig == 0 || ma.n_dig > kMfMaxDigits || ma.n_grp == 0) return hipErrorInvalidValue;
     // algorithmic bytes: inputs read once, outputs written
     double limbs = 0;
-    for (uint32_t d = 0; d < ma.n_dig; d++) limbs += ma.dig[d].n_in + ma.dig[d].n_out + (extra ? 1 : 0);
-    const int pi = prof_begin(ctx, name, limbs * B * kN * 8, st);
-    const dim3 grid(256 / kBcWaves * ma.n_grp * B), block(64 * kBcWaves);
     bool tail = true;
     for (uint32_t d = 0; d < ma.n_dig; d++) {
         if (ma.dig[d].n_in == 0 || ma.dig[d].n_in > 8 * ks) return hipErrorInvalidValue;
         tail = tail && ma.dig[d].n_in <= 9;
+        limbs += ma.dig[d].n_in + ma.dig[d].n_out + (extra ? 1 : 0);
     }
+    const int pi = prof_begin(ctx, name, limbs * B * kN * 8, st);
+    const dim3 grid(256 / kBcWaves * ma.n_grp * B), block(64 * kBcWaves);
     auto k = ks == 1 ? (extra ? k_bconv_ntt_a<1, false, true> : k_bconv_ntt_a<1, false, false>)
              : tail  ? (extra ? k_bconv_ntt_a<2, true, true> : k_bconv_ntt_a<2, true, false>)
                      : (extra ? k_bconv_ntt_a<2, false, true> : k_bconv_ntt_a<2, false, false>);
