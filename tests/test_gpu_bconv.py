@@ -1,6 +1,6 @@
 """GPU parity of the basis conversions (ModUp, ModDown with and without the rescale, both roundings) over the shapes that
 their matrix-core form splits by: source limbs in steps of 8 (with one left over, or more), outputs in groups of four (the
-last one padded), primes of 34 to 60 bits mixed in a chain, and chains with smaller primes, which take the other form.
+last one padded), primes of 36 to 60 bits mixed in a chain, and chains with smaller primes, which take the other form.
 Every value is an integer residue: the words must equal the CPU oracle's."""
 import numpy as np
 import pytest
@@ -18,7 +18,8 @@ def ckks():
 
 
 def residues(moduli, shape_prefix, prime_idx, seed):
-    """uniform residues; the first words of every limb are 0, 1, q - 1 and digit edges (0x7f.., 0x80..)"""
+    """uniform residues; the first words of every limb are 0, 1, q - 1, 0x7f.. and 0x80.. (evaluation form: what the
+    conversions read is an inverse NTT of these; test_gpu_conversion_extremes.py forms their own extremes)"""
     rng = np.random.default_rng(seed)
     q = np.array([moduli[i] for i in prime_idx], dtype=np.uint64)
     x = rng.integers(0, 2**63, tuple(shape_prefix) + (len(prime_idx), N), dtype=np.uint64)

@@ -86,3 +86,49 @@ def test_both_forms_bit_exact_at_the_lines(ckks, oracle, chain, exact, n):
             assert all(np.array_equal(g, want) for g in dm.download((n, 2, l - 1, N))), (l, "product")
             assert head == head_expected("product", l, n, K), (l, "product's form")
     ctx.close()
+
+
+@pytest.mark.parametrize("exact", [False, True])
+@pytest.mark.parametrize("shape", [(16, 2, 8, (16, 13, 9)), (6, 2, 6, (6, 5))])
+def test_five_to_eight_digits_bit_exact(ckks, oracle, shape, exact):
+    """more than four digits: the inner products and the addend's dropped limb take launches of their own, in both forms
+    (at the first chain's upper levels the matrix cores, whose limbs are column-major within 16 rows)"""
+    L, K, dnum, levels = shape
+    ctx = ckks.Context(num_q=L, num_p=K, dnum=dnum, q_bits=54, p_bits=60)
+    ctx.set_moddown_exact(exact)
+    oc = oracle.Ctx(16, ctx.moduli, L, K, dnum, moddown_exact=exact)
+    evk = residues(ctx.moduli, (dnum, 2), list(range(L + K)), 3)
+    devk = ckks.DeviceBuffer.from_array(evk)
+    for l in levels:
+        D, E, n = ctx.num_digits(l), l + K, 2
+        print(f"{D} digits at level {l}, {'exact' if exact else 'approximate'}", flush=True)
+        assert D > 4
+        x = residues(ctx.moduli, (n,), list(range(l)), 10 + l)
+        dx, dext = ckks.DeviceBuffer.from_array(x), ckks.DeviceBuffer(n * D * E * N * 8)
+        ctx.modup(dx.ptr, n, l, dext.ptr)
+        ext = dext.download((n, D, E, N))
+        dks = ckks.DeviceBuffer(n * 2 * l * N * 8)
+        ctx.keyswitch(dx.ptr, n, l, devk.ptr, dks.ptr)
+        ks = dks.download((n, 2, l, N))
+        for i in range(n):
+            assert np.array_equal(ext[i], oc.modup(x[i], l)), (l, i, "ModUp")
+            assert np.array_equal(ks[i], oc.keyswitch(x[i], l, evk)), (l, i, "key switch")
+        a, b = (residues(ctx.moduli, (n, 2), list(range(l)), 30 + l + s) for s in (0, 1))
+        da, db = ckks.DeviceBuffer.from_array(a), ckks.DeviceBuffer.from_array(b)
+        steps, drot = [1, -3], ckks.DeviceBuffer(2 * 2 * l * N * 8)
+        ctx.eval_rotate_hoisted(da.ptr, l, steps, [devk.ptr, devk.ptr], drot.ptr)
+        rot = drot.download((2, 2, l, N))
+        for i, s in enumerate(steps):
+            assert np.array_equal(rot[i], oc.rotate(a[0], l, oc.rot_index(s), evk)), (l, s, "rotation")
+        dm = ckks.DeviceBuffer(n * 2 * (l - 1) * N * 8)
+        ctx.eval_mult_rescale(da.ptr, db.ptr, n, l, devk.ptr, dm.ptr)
+        got = dm.download((n, 2, l - 1, N))
+        want = [oc.hmult_relin_rescale(a[i], b[i], l, evk) for i in range(n)]
+        assert all(np.array_equal(got[i], want[i]) for i in range(n)), (l, "product")
+        ctx.eval_mult_sum([[(da.ptr, db.ptr)]], l, devk.ptr, dm.ptr)
+        assert np.array_equal(dm.download((2, l - 1, N)), want[0]), (l, "sum of products")
+        # in place: the combine may not read the inputs again
+        ctx.eval_mult_rescale(da.ptr, db.ptr, n, l, devk.ptr, da.ptr)
+        got = da.download((n, 2, l - 1, N))
+        assert all(np.array_equal(got[i], want[i]) for i in range(n)), (l, "product in place")
+    ctx.close()
