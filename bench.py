@@ -90,26 +90,17 @@ def achievable(write_share: float) -> float:
 #            reads off the two counters); for ("workload", "step") summed over every dispatch of one step;
 #   valu:    wave64 VALU instructions issued (SQ_INSTS_VALU, all waves of the launch).
 # A kernel "launch" is one engine call (both kernels of a two-pass NTT).  Measured, not computed: re-measure when the
-# kernel or the workload changes.  The step figures of pcmm, bootstrap and decode are of the kernels before the
-# matrix-core basis conversion: the bench line leaves their traffic out until it is counted again.
+# kernel or the workload changes.  The forward NTTs that follow a basis conversion are their second passes alone.
 MEASURED = {
-    ("hmult", "step"): {"traffic": 33.103e9, "source": "profiles/hmult_config2_kernels.md"},
-    ("hmult", "ntt_fwd_mdr"): {"traffic": 10.905e9, "valu_insts": 879.5e6, "source": "profiles/hmult_config2_kernels.md"},
-    ("hmult", "ntt_fwd_2pass"): {"traffic": 9.700e9, "valu_insts": 776.7e6, "source": "profiles/hmult_config2_kernels.md"},
-    # the same workload with the matrix-core basis conversion (the kernels the bench runs now): the forward NTTs that follow
-    # a conversion are their second passes alone
-    ("hmult_mfma", "step"): {"traffic": 25.859e9, "source": "profiles/hmult_matrix_core_kernels.md"},
-    ("hmult_mfma", "ntt_fwd_mdr"): {"traffic": 7.814e9, "valu_insts": 662.5e6,
-                                    "source": "profiles/hmult_matrix_core_kernels.md"},
-    ("hmult_mfma", "ntt_fwd_2pass"): {"traffic": 4.865e9, "valu_insts": 403.9e6,
-                                      "source": "profiles/hmult_matrix_core_kernels.md"},
-    ("hmult_mfma", "bconv"): {"traffic": 3.223e9, "valu_insts": 450.9e6,
-                              "source": "profiles/hmult_matrix_core_kernels.md"},
+    ("hmult", "step"): {"traffic": 25.862e9, "source": "profiles/hmult_config2_kernels.md"},
+    ("hmult", "ntt_fwd_mdr"): {"traffic": 7.816e9, "valu_insts": 662.5e6, "source": "profiles/hmult_config2_kernels.md"},
+    ("hmult", "ntt_fwd_2pass"): {"traffic": 4.866e9, "valu_insts": 403.9e6, "source": "profiles/hmult_config2_kernels.md"},
+    ("hmult", "bconv"): {"traffic": 3.223e9, "valu_insts": 450.9e6, "source": "profiles/hmult_config2_kernels.md"},
     ("ntt", "step"): {"traffic": 12.940e9, "source": "profiles/ntt_config1_kernel_trace.md"},
-    ("pcmm", "step"): {"traffic": 18.373e9, "source": "profiles/pcmm_config3_kernel_trace.md"},
-    ("pcmm", "bsgs_mac"): {"traffic": 7.382e9, "source": "profiles/pcmm_config3_kernel_trace.md"},
-    ("bootstrap", "step"): {"traffic": 53.876e9, "source": "profiles/bootstrap_config4_kernel_trace.md"},
-    ("decode", "step"): {"traffic": 21302.8e9, "source": "profiles/decode_config5_kernel_trace.md"},
+    ("pcmm", "step"): {"traffic": 16.508e9, "source": "profiles/pcmm_config3_kernel_trace.md"},
+    ("pcmm", "bsgs_mac"): {"traffic": 7.383e9, "source": "profiles/pcmm_config3_kernel_trace.md"},
+    ("bootstrap", "step"): {"traffic": 48.248e9, "source": "profiles/bootstrap_config4_kernel_trace.md"},
+    ("decode", "step"): {"traffic": 18173.6e9, "source": "profiles/decode_config5_kernel_trace.md"},
     ("ntt", "ntt_fwd_2pass"): {"traffic": 6.470e9, "valu_insts": 480.5e6, "source": "profiles/ntt_config1_kernel_trace.md"},
     ("ntt", "ntt_inv_2pass"): {"traffic": 6.470e9, "valu_insts": 482.3e6, "source": "profiles/ntt_config1_kernel_trace.md"},
 }
@@ -233,10 +224,10 @@ def bench_hmult(ckks, torch, steps, warmup, seed):
                    "step_ms_min": round(min(per), 4), "step_ms_max": round(max(per), 4)},
         "check": {"decrypted_relErrRms_max": rel_err, "ciphertexts_checked": 2},
         "kernels": kernel_table(rep),
-        "roofline": step_roofline("hmult_mfma", N_PAIRS * HMULT_UNIT_BYTES, step_ms, 46 / 334,
+        "roofline": step_roofline("hmult", N_PAIRS * HMULT_UNIT_BYTES, step_ms, 46 / 334,
                                   "step: one ckks_eval_mult_rescale call over 64 pairs; SURVEY 8(d) config-2 unit "
                                   "175,112,192 B per op (inputs 96 + evk 192 + output 46 limbs) x 64"),
-        "kernel_io": kernel_io(rep, "hmult_mfma"),
+        "kernel_io": kernel_io(rep, "hmult"),
         "ks_stage": ks_stage(rep, step_ms),
     }
     res["roofline"]["evk_amortised"] = step_roofline(
@@ -382,7 +373,7 @@ def bench_pcmm(ckks, torch, steps_n, warmup, seed):
     alg = ((len(bst) + len(gst)) * 96 + d * l + 62) * LIMB_BYTES
     return {"ms_per_pcmm": round(ms, 4), "relErrRms_vs_fp64": rel,
             "kernels": kernel_table(rep), "kernel_io": kernel_io(rep, "pcmm"),
-            "roofline": step_roofline("", alg, ms, 30 / (alg / LIMB_BYTES),
+            "roofline": step_roofline("pcmm", alg, ms, 30 / (alg / LIMB_BYTES),
                                       f"step: one ckks_linear_transform_bsgs call; SURVEY 8(d) config-3 unit with "
                                       f"{len(bst) + len(gst)} keys: keys + 768 x 16 diagonal limbs + ct in/out"),
             "workload": "config3: 768x768 fp64 weights N(0,1/768) x 1 ct at L=16, BSGS 28 baby x 28 giant, "
@@ -479,7 +470,7 @@ def bench_bootstrap(ckks, torch, steps_n, warmup, seed, form="sparse_r2", stage_
     return {"ms_per_bootstrap": round(ms, 3), "precision_bits": round(bits, 2),
             "levels_in_out": [1, bt.out_level], "rotation_keys": len(bt.steps), "stage_errors": stages,
             "form": form, "kernels": kernel_table(rep), "kernel_io": kernel_io(rep, "bootstrap"),
-            "roofline": step_roofline("", profile_bytes(rep), ms, 0.5,
+            "roofline": step_roofline("bootstrap" if form == "sparse_r2" else "", profile_bytes(rep), ms, 0.5,
                                       "step: one ckks_eval_bootstrap call; SURVEY 8(d) config-4 unit: the sum of its "
                                       "launches' algorithmic bytes (each launch's inputs, keys, diagonals and outputs "
                                       "once)"),
@@ -636,7 +627,7 @@ def bench_decode(ckks, torch, steps_n, warmup, seed, n_layers=12, driver="native
             "client_s": {"decrypt_and_vocab_head": round(t_client, 3)},
             "kernels": kernel_table(rep), "kernel_io": kernel_io(rep, "decode"),
             "phases": phase_table(phases, s_per_step * 1e3), "phase_marker_ids": marker_ids,
-            "roofline": step_roofline("", profile_bytes(rep), s_per_step * 1e3, 0.5,
+            "roofline": step_roofline("decode", profile_bytes(rep), s_per_step * 1e3, 0.5,
                                       "step: one decode step of the native driver; SURVEY 8(d) config-5 unit: the sum "
                                       "of its launches' algorithmic bytes (each launch's inputs, keys, diagonals and "
                                       "outputs once)"),
