@@ -24,10 +24,11 @@
 // consecutive bytes: with row-major limbs and workgroup tiles of 8 columns, whose 64-byte pieces of lines cost full ones,
 // the same conversion took 1,515 us.
 //
-// Measured (64 x 3 digits, 8 -> 24 limbs of 54 and 60 bits): 1,125 us, where the conversion on the VALU (739 us, VALU-bound)
-// and the separate first pass (974 us) took 1,713; 128 ModDowns of 8 -> 23 limbs 827 us and their head 163, before 569 and
-// 669.  What bounds it: 476 M VALU wave instructions (71 of the 100 an output word are the butterflies), 0.85 ms at the
-// issue rate, over 3.2 GB of memory traffic.
+// Measured (64 x 3 digits, 8 -> 24 limbs of 54 and 60 bits): 1,093-1,178 us, where the conversion on the VALU (739 us,
+// VALU-bound) and the separate first pass (974 us) took 1,713; 128 ModDowns of 8 -> 23 limbs 811-882 us and their head
+// 146-152, before 569 and 669.  What bounds it: 451 M VALU wave instructions (71 of the 96 an output word are the
+// butterflies), 0.96 ms at the issue rate of the 1.84 GHz that it holds, over 3.2 GB of memory traffic.  With few outputs
+// the VALU form is the faster one: the rule and its measurements are at mf_modup and mf_moddown in ops.cpp.
 #include <algorithm>
 
 #include "bconv_ntt.hpp"
@@ -186,11 +187,10 @@ __device__ __forceinline__ void bc_column(const uint64_t* __restrict__ in, const
     sh.tw[lane] = tv;
     wave_exchange();
     stages03<kOpen>(x, sh.tw + 16 * g, c.q);
-    // rows 16 n + k: the twiddles of stages 4..6 are requested before the exchange, stage 7's after it.  Stage s's
-    // entry
+    // rows 16 n + k: the twiddles of stages 4..6 are requested before the exchange, stage 7's after it.  Stage s's entry
     // 2^s + 2^(s-4) n + j of the plain table stands at 2^s + 16 j + n of this kernel's (twa), so that a load's 16 lanes of
-    // an output read 256 consecutive bytes (in the plain table stage 7's lanes are a line apart,
-    // and the loads took a fifth of the kernel's time)
+    // an output read 256 consecutive bytes (in the plain table stage 7's lanes are a line apart, and the loads took a fifth
+    // of the kernel's time)
     const TwPair* tw = twa + 256 * c.prime + n;
     TwPair tw47[15];
 #pragma unroll
@@ -219,9 +219,11 @@ __device__ __forceinline__ void bc_column(const uint64_t* __restrict__ in, const
 
 // grid: 64 quads of columns x (groups of 4 outputs of every digit) x batch, one dimension.  Workgroups go to the 8 XCDs
 // round-robin; id = xcd + 8 s, and XCD xcd takes the columns [32 xcd, 32 xcd + 32), s running over their 8 quads fastest,
-// then the groups (which read the same source words, kept by that XCD's L2), then the batch.  Two steps of source limbs
-// take 136 registers: three waves a SIMD without spills and 8 rows' words in flight (11 conversions of 9 -> 25 limbs
-// 436 us) against four with 3 spilled and 4 rows' (464).
+// then the groups (which read the same source words, kept by that XCD's L2), then the batch.
+// Two steps of source limbs run three waves a SIMD with 8 rows' words in flight: 140 to 156 registers, and 168 with 3
+// spilled for 10 to 16 limbs with an added one; four waves with 4 rows' have 128 and spill 3 to 10.  Three against four, us
+// (whole levels of 54- and 60-bit chains, 16 x 2 digits or 32 ModDowns): 16 limbs 337 / 361 ModUp, 314 / 319 ModDown, 311-324
+// / 346 exact; 12 limbs 256 / 272, 234 / 236, 226-237 / 253; 9 limbs 197-202 / 202, 179 / 179, 168 / 162.
 template <int KS, bool kTail, bool kExtra>
 __global__ __launch_bounds__(64 * kBcWaves) __attribute__((amdgpu_waves_per_eu(KS == 2 ? 3 : 4))) void k_bconv_ntt_a(
     const uint64_t* __restrict__ in, const uint64_t* __restrict__ extra, uint64_t* __restrict__ out, MfArgs ma,

@@ -1262,8 +1262,9 @@ hipError_t launch_ntt_fwd_b(const Context& ctx, uint64_t* data, const JobSpec& j
     return hipGetLastError();
 }
 
-// a_done (the launchers that end in a combine): the buffer already holds the first pass's output as the basis conversion
+// In the launchers that end in a combine, a_done: the buffer already holds the first pass's output as the basis conversion
 // leaves it (bconv_ntt.hip: tiles of 16 blocks column-major); the second pass alone is launched.
+
 // launch_ntt_inv_ks for a key-switch list of n items (item c: extension ext[c] [D][E][N], key evk[c])
 hipError_t launch_ntt_inv_ksl(const Context& ctx, uint64_t* acc, const JobSpec& js, uint32_t n_jobs,
                               const uint64_t* const* ext, const uint64_t* const* evk, uint32_t n, uint32_t D,

@@ -1115,8 +1115,9 @@ void hmult(Context& ctx, const uint64_t* a, const uint64_t* b, uint32_t B, uint3
         relin_tail(ctx, d01, x2c, ext, B, l, evk, out, do_rescale, st, nullptr, nullptr, true, aff);
 }
 
-// Device workspace of hmult with the rescale (bytes): d01 2Bl, d2 Bl, extension B D E, inner product 2B E,
-// the addend's dropped limb 2B and the rescale's T 2B (l-1) limbs
+// Device workspace of hmult with the rescale (bytes): d01 2Bl, d2 Bl, extension B D E, inner product 2B E, the rescale's T
+// 2B (l-1) limbs, and 2B of the addend's dropped limb, which has a buffer under the fused NTT mode or with more than 4
+// digits only: the bound (and so the largest batch of the allocation-free entry) is one for all of them
 size_t hmult_rescale_scratch_bytes(const Context& ctx, uint32_t B, uint32_t l) {
     const size_t D = num_digits(ctx, l), E = l + ctx.K;
     const size_t limbs = (size_t)B * (2 * l + l + D * E + 2 * E + 2 + 2 * (l - 1));

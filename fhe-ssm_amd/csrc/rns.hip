@@ -105,7 +105,8 @@ __global__ __launch_bounds__(256) void k_tensor_sum(const uint64_t* const* __res
 // in  : batch c -> in + c*in_bstride, source limb i at off(in_desc[i])*N, prime prime(in_desc[i])
 // out : batch c -> out + c*out_bstride, target limb j at off(out_desc[j])*N, prime prime(out_desc[j])
 // tab : [n_in] TwPair (qhinv, companion) followed by [n_in][n_out] uint64 qhmod
-// Used where the matrix-core form (bconv_ntt.hip) is not: under the fused NTT mode, and for chains with a prime below 2^34.
+// Used where the matrix-core form (bconv_ntt.hip) is not: under the fused NTT mode, for chains with a prime below 2^34, for
+// ModUps to more than 80 limbs of Q_l P, and for few outputs (mf_modup, mf_moddown in ops.cpp).
 // Every BConv output is the input of a forward NTT, which takes words below 8q and stores canonical residues: the
 // Montgomery-reduced instances leave their outputs in [0, 2q) (redc_lazy), skipping the final conditional
 // subtraction; the ModDown+rescale instance adds the rescale's lift to that, below q (lift_centered) or below 3q (the
