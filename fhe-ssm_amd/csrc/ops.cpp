@@ -415,13 +415,13 @@ static bool mf_modup(const Context& ctx, uint32_t l, uint32_t B) {
 // ModDown to l limbs of n_polys polys.
 static bool mf_moddown(const Context& ctx, uint32_t kind, uint32_t l, uint32_t n_polys, bool list) {
     if (ctx.ntt_mode != NttMode::TwoPass || !ctx.mf_primes || ctx.K > (uint32_t)kMfMaxIn || l > kMfMaxOut) return false;
-    // with the rescale: K = 8, product of 32 pairs to 2 limbs +8%, 4 limbs +4%, 8 limbs +-1%, 16 limbs -2%, 24 -3%; of one
-    // pair 2 limbs +-1%, 5 limbs -3%, 24 limbs -10%
-    if (kind == kMfDownRescale) return l >= (n_polys >= 16 ? 8u : 3u);
+    // with the rescale, whole products (mean of K = 2, 4, 6, 8, 12): 4 pairs 2 limbs +1%, 3 limbs -1%; 6 pairs 3 limbs +2%; 16
+    // pairs 4 limbs +-0, 5 limbs -1%, 6 limbs +-0; 28 pairs 6 limbs +3%, 7 limbs +-0, 9 limbs -2%; of one pair 24 limbs -10%
+    if (kind == kMfDownRescale) return l >= (n_polys <= 8 ? 3u : n_polys <= 32 ? 5u : 7u);
     if (ctx.moddown_exact) {
-        // of a key-switch list: K = 8, 32 items 3 limbs +6%, 6 limbs +2%, 8 limbs -1%, 24 limbs -4%; one item 2 limbs +1%,
-        // 4 limbs -2%
-        if (list) return l >= (n_polys > 16 ? 8u : 4u);
+        // of a key-switch list (the same mean): one item 3 limbs +1%, 4 limbs -1%; 12 items 4 limbs -2%, 5 limbs +1%, 6 limbs
+        // -2%; 20 items 5 limbs +3%, 6 limbs -1%; 28 items 6 limbs +1%, 7 limbs -2%
+        if (list) return l >= (n_polys <= 24 ? 4u : n_polys <= 48 ? 6u : 7u);
         // alone: K = 8, 2 polys 8 limbs +7%, 11 limbs +5%, 16 limbs -7%; 8 polys 4 limbs +-0, 8 limbs -3%; 64 polys 5 limbs
         // +8%, 8 limbs -1%; K = 2, 8 polys 8 limbs +6%, 11 limbs +1%, 24 polys 8 limbs -6%
         return l >= 12 || (l >= 8 && n_polys * ctx.K >= 48);

@@ -28,18 +28,18 @@ def residues(moduli, shape_prefix, prime_idx, seed):
 # name: (Q limbs, special primes, dnum)
 CHAINS = {"one special prime": (4, 1, 4), "two special primes": (12, 2, 4), "eight special primes": (13, 8, 2)}
 # level -> polys of a lone exact ModDown, items of a key-switch list, pairs of a product that take the matrix cores
-LEVELS = (1, 2, 3, 4, 7, 8, 12)
+LEVELS = (1, 2, 3, 4, 5, 6, 7, 8, 12)
 
 
 def head_expected(what, l, n, K):
     if what == "moddown":
         return l >= 12 or (l >= 8 and n * K >= 48)
     if what == "list":
-        return l >= (8 if 2 * n > 16 else 4)
-    return l >= (8 if 2 * n >= 16 else 3)  # a product with its rescale
+        return l >= (4 if n <= 12 else 6 if n <= 24 else 7)
+    return l >= (3 if n <= 4 else 5 if n <= 16 else 7)  # a product with its rescale
 
 
-@pytest.mark.parametrize("n", [1, 9])
+@pytest.mark.parametrize("n", [1, 5, 13, 25])
 @pytest.mark.parametrize("exact", [False, True])
 @pytest.mark.parametrize("chain", sorted(CHAINS))
 def test_both_forms_bit_exact_at_the_lines(ckks, oracle, chain, exact, n):
